@@ -172,7 +172,10 @@ void ufomi_bp_params_init(ufomi_bp_params *p);
  * half-precision (v, d) staging interpolated with v_dot2_f32_f16 (half the
  * LDS bytes; adds one f16 rounding of the sample difference and of the
  * weight): 0 or positive = on (the default), negative = off.  Slices and
- * chunk do not change results; half staging does.  No counterpart in the
+ * chunk do not change results; half staging does.  With both automatic,
+ * stacks of 12 and more slices with enough work run on the matrix cores
+ * (two-term f16 samples and weights, f32 sums, 22-bit samples: the same result
+ * up to rounding), which asks for no configuration.  No counterpart in the
  * reference.
  */
 int ufomi_bp_configure(ufomi_ctx *ctx, int slices_per_tile, int angle_chunk, int half_staging);
@@ -190,8 +193,9 @@ int ufomi_bp_parallel(ufomi_ctx *ctx, const void *d_sino, int dtype, int W, int 
                       float *d_out, size_t out_slice_pitch);
 
 /*
- * ufomi_bp_parallel without any device allocation: same arguments, kernels
- * and results, but the (sin, cos) table (computed on the device in FP64 and
+ * ufomi_bp_parallel without any device allocation: same arguments and
+ * results (up to rounding for stacks, which keep the interpolating kernel
+ * here: the matrix-core path needs a workspace), but the (sin, cos) table (computed on the device in FP64 and
  * rounded to float, as the LUT of ufomi_bp_parallel) and the partial volumes
  * of an angle split live in one preallocated array per GPU (64.25 MiB, held
  * until the process ends), and no host-to-device copy is made.  It has no

@@ -1,0 +1,151 @@
+"""Stacks of slices on the matrix cores (bp_mfma.hip) against the oracle and the interpolating kernel.
+
+The path takes 12 and more slices with at least 1e9 updates (2.5e9 in f16 storage), in units of 64, 32
+and 16 slices with up to 8 leftover ones on the interpolating kernel, four angles at a time on 32 x 32
+tiles.  Bars: 1e-5 relative L2, the bar of the interpolating kernel (float32 coordinates of up to 512
+pixels round at 3e-5 pixels); 16-bit storage is compared on the stored values, so the same bar holds.
+"""
+import numpy as np
+import pytest
+
+import oracle
+import ufomi
+from conftest import rel_l2
+
+pytestmark = pytest.mark.gpu
+DTYPES = {"f32": (ufomi.F32, "float32"), "f16": (ufomi.F16, "float16"), "bf16": (ufomi.BF16, "bfloat16")}
+
+
+def _both(ctx, torch_dev, x, storage="f32", **props):
+    """(matrix cores, interpolating kernel) results of stack x [S][P][W]."""
+    import torch
+    S, P, W = x.shape
+    code = DTYPES[storage][0]
+    rw, rh = props.get("roi_width") or W, props.get("roi_height") or W
+    outs = []
+    try:
+        for config in ((0, 0, 0), (8, 8, -1)):
+            ctx.bp_configure(*config)
+            out = torch.full((S, rh, rw), float("nan"), device=torch_dev)
+            ctx.bp_parallel(x, W, P, out, n_slices=S, dtype=code, **props)
+            outs.append(out)
+    finally:
+        ctx.bp_configure(0, 0, 0)
+    return outs
+
+
+def _stack(torch_dev, S, P, W, storage="f32", seed=1):
+    import torch
+    x = np.random.default_rng(seed).standard_normal((S, P, W)).astype(np.float32)
+    return torch.from_numpy(x).to(torch_dev).to(getattr(torch, DTYPES[storage][1]))
+
+
+@pytest.mark.parametrize("S,P,W,storage", [
+    (12, 401, 480, "f32"), (16, 402, 400, "f32"), (17, 403, 400, "f32"), (32, 300, 351, "f32"),
+    (33, 300, 352, "f32"), (41, 260, 321, "f32"), (48, 200, 353, "f32"), (49, 200, 353, "f32"),
+    (64, 129, 383, "f32"), (73, 1, 3800, "f32"), (130, 64, 512, "f32"),
+    (20, 500, 511, "f16"), (64, 400, 320, "f16"), (40, 300, 333, "bf16"),
+])
+def test_units_vs_oracle(ctx, torch_dev, S, P, W, storage):
+    """Full and padded units of 64, 32 and 16 slices, leftovers, angle counts off the fours, split and
+    unsplit angles, widths off the tiles.  Against FP64 the bar is the rounding of the inputs of both kernels:
+    the float32 (sin, cos) table is off by up to 3e-8, which at 0.7 W (360 pixels) moves a sample by up to 1e-5
+    pixels, and white noise turns that into the same relative error; the axis is a float32 number."""
+    x = _stack(torch_dev, S, P, W, storage, seed=S)
+    got, ref = _both(ctx, torch_dev, x, storage, axis_pos=W / 2.0 + 0.25)
+    got, ref = got.cpu().numpy(), ref.cpu().numpy()
+    assert np.isfinite(got).all()
+    for s in range(S):
+        assert rel_l2(got[s], ref[s]) < 1e-5, s
+    s = S // 2
+    if W < 1000:
+        exact = oracle.bp_texture_f64(x[s].float().cpu().numpy(), axis_pos=W / 2.0 + 0.25)
+        assert rel_l2(got[s], exact) < 1e-5
+        assert rel_l2(got[s], exact) < 1.2 * rel_l2(ref[s], exact) + 1e-7  # no less precise
+
+
+@pytest.mark.parametrize("props", [
+    dict(axis_pos=150.25, roi_x=33, roi_y=7, roi_width=301, roi_height=215, angle_offset=0.7),
+    dict(angle_step=0.013, offset=11, num_projections=700),
+    dict(axis_pos=1.5, roi_width=420, roi_height=300),   # most of the image off the detector
+])
+def test_geometry_and_pitches(ctx, torch_dev, props):
+    import torch
+    S, P, W = 24, 600, 300
+    x = _stack(torch_dev, S, P, W, seed=5)
+    rw, rh = props.get("roi_width") or W, props.get("roi_height") or W
+    wide = torch.zeros((S, P * W + 37), device=torch_dev)
+    wide[:, :P * W] = x.view(S, -1)
+    pitch = rw * rh + 3  # slices of the output off the 16-byte alignment
+    got, _ = _both(ctx, torch_dev, x, "f32", **props)
+    flat = []
+    for config in ((0, 0, 0), (8, 8, -1)):
+        try:
+            ctx.bp_configure(*config)
+            out = torch.full((S, pitch), 7.0, device=torch_dev)
+            ctx.bp_parallel(wide, W, P, out, n_slices=S, sino_pitch=P * W + 37, out_pitch=pitch, **props)
+            flat.append(out.cpu().numpy())
+        finally:
+            ctx.bp_configure(0, 0, 0)
+    assert (flat[0][:, rw * rh:] == 7.0).all()  # nothing past a slice
+    assert rel_l2(flat[0][:, :rw * rh], flat[1][:, :rw * rh]) < 1e-5
+    np.testing.assert_array_equal(flat[0][:, :rw * rh].reshape(S, rh, rw), got.cpu().numpy())
+
+
+@pytest.mark.parametrize("storage", ["f32", "f16", "bf16"])
+def test_nonfinite_values_stay_local(ctx, torch_dev, storage):
+    """An Inf or a NaN reaches the pixels whose samples touch it and no others, whichever unit it is in."""
+    import torch
+    x = _stack(torch_dev, 105, 300, 300, storage, seed=7)
+    x[3, 150, 140] = float("inf")
+    x[70, 0, 1] = float("nan")
+    x[100, 299, 299] = float("-inf")
+    got, ref = _both(ctx, torch_dev, x, storage)
+    assert bool((torch.isfinite(got) == torch.isfinite(ref)).all())
+    assert bool((torch.isnan(got) == torch.isnan(ref)).all())
+    m = torch.isfinite(ref)
+    assert float((got[m] - ref[m]).norm() / ref[m].norm()) < 1e-5
+
+
+def test_scales(ctx, torch_dev):
+    """Slices of very different size each keep their precision, denormal and all-zero ones too."""
+    import torch
+    x = _stack(torch_dev, 16, 400, 400, seed=9)
+    scale = [1.0, 1e-30, 1e30, 1e-20, 0.0, 65504.0, 1e-38, 3e-41, 2.0 ** -14, 1e10, 1e-5, 1e5, 1.0, 1e35, 1e-36, 7.0]
+    x *= torch.tensor(scale, device=torch_dev)[:, None, None]
+    got, ref = _both(ctx, torch_dev, x)
+    got, ref = got.cpu().numpy().astype(np.float64), ref.cpu().numpy().astype(np.float64)
+    for s, v in enumerate(scale):
+        if v == 0.0:
+            assert (got[s] == 0.0).all()
+        elif v >= 1e-36:
+            assert rel_l2(got[s], ref[s]) < 1e-5, v
+        else:  # results near the smallest normal float: half a denormal step (7e-46) per addition at most
+            assert np.abs(got[s] - ref[s]).max() < 400 * 1.5e-45, v
+
+
+def test_streams_share_a_context(ctx, torch_dev):
+    """Calls of one context on two streams in turn: the second waits for the first one's workspace."""
+    import torch
+    a, b = _stack(torch_dev, 64, 400, 512, seed=1), _stack(torch_dev, 48, 300, 400, seed=2)
+    oa, ob = torch.empty((64, 512, 512), device=torch_dev), torch.empty((48, 400, 400), device=torch_dev)
+    ctx.bp_parallel(a, 512, 400, oa, n_slices=64)
+    ctx.bp_parallel(b, 400, 300, ob, n_slices=48)
+    torch.cuda.synchronize()
+    ra, rb = oa.clone(), ob.clone()
+    side = torch.cuda.Stream()
+    main = torch.cuda.current_stream(0)
+    side.wait_stream(main)
+    try:
+        for _ in range(4):
+            oa.zero_()
+            ctx.set_stream(main)
+            ctx.bp_parallel(a, 512, 400, oa, n_slices=64)
+            ctx.set_stream(side)
+            with torch.cuda.stream(side):
+                ob.zero_()
+                ctx.bp_parallel(b, 400, 300, ob, n_slices=48)
+            torch.cuda.synchronize()
+            assert torch.equal(oa, ra) and torch.equal(ob, rb)
+    finally:
+        ctx.set_stream(main)

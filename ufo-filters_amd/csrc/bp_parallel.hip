@@ -6,8 +6,10 @@
 // 8-bit weights, too coarse for 1e-5 parity, so interpolation is done in
 // float32 in registers from LDS:
 //
+// Stacks of 12 and more slices run on the matrix cores instead (bp_mfma.hip).
+//
 //  * A 256-thread workgroup owns a 32x32 voxel tile of S slices that share the
-//    geometry (S = 1, 2 or 4).  Thread (lx, ly) owns voxels
+//    geometry (S = 1, 2, 4 or 8).  Thread (lx, ly) owns voxels
 //    (lx + 16 kx, ly + 16 ky), kx, ky in {0, 1}; a wave covers 16x4 adjacent
 //    voxels, so its 64 LDS reads fall inside ~18 consecutive entries.
 //  * Angles are processed in chunks of A = 16.  For every angle of a chunk the
@@ -419,6 +421,28 @@ bp_texture_kernel(const InT *__restrict__ sino, long sino_pitch, int W, int P, c
                                    roi_h, n_slices, g * S, o, out_pitch, tx * kTile, ty * kTile, P);
 }
 
+// The tiles of bp_texture_kernel<8, 8> for the units of slices of which one holds an Inf or a NaN
+// (maxbits, the bits of a slice's largest |v|): units of 64 slices up to slice n64, of 32 up to n32,
+// of 16 after.  The other units are skipped.
+template <typename InT>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) void bp_nonfinite_kernel(
+    const InT *__restrict__ sino, long sino_pitch, int W, int P, const float2 *__restrict__ trig, float axis,
+    float roi_x, float roi_y, int roi_w, int roi_h, int n_slices, int n64, int n32,
+    const unsigned *__restrict__ maxbits, float *__restrict__ out, long out_pitch, int tiles_x, int tiles)
+{
+    for (int u0 = 0, unit; u0 < n_slices; u0 += unit) {
+        unit = u0 < n64 ? 64 : u0 < n32 ? 32 : 16;
+        const int s = min(u0 + (int) (threadIdx.x & 63), min(u0 + unit, n_slices) - 1);
+        if (!__ballot(maxbits[s] >= 0x7f800000u)) continue;  // the same in every wave
+        for (long w = blockIdx.x; w < (long) tiles * (unit / 8); w += gridDim.x) {
+            const int g = u0 + 8 * (int) (w / tiles), t = (int) (w % tiles);
+            if (g < n_slices)
+                bp_tile<8, kTile, 8, InT>(sino, sino_pitch, W, P, trig, axis, roi_x, roi_y, roi_w, roi_h, n_slices, g,
+                                          out, out_pitch, (t % tiles_x) * kTile, (t / tiles_x) * kTile);
+        }
+    }
+}
+
 // Sum of the partial volumes of an angle-split launch, in split order.
 __global__ __launch_bounds__(kThreads) void bp_sum_parts_kernel(const float *__restrict__ part, int n_split,
                                                                 long part_stride, long plane, int n_slices,
@@ -692,6 +716,26 @@ int bp_parallel_impl(ufomi_ctx *ctx, const void *d_sino, int dtype, int W, int P
     if (prm->mode != UFOMI_BP_TEXTURE)
         return ufomi_fail(UFOMI_ERR_ARG, "unknown backprojection mode %d", prm->mode);
 
+    // Stacks go to the matrix cores (bp_mfma.hip) unless a tile configuration is asked for; up to
+    // 8 slices that would fill less than half a unit there stay here.  Below 12 slices a unit is
+    // mostly padding.  The scaled copy of the rows and its four launches cost 30-60 us: measured in
+    // us, this kernel / the matrix cores, f32 storage: 24 slices of 400^2 x 180 (6.9e8 updates)
+    // 100 / 102, 12 of 400^2 x 500 (9.6e8) 162 / 132, 64 of 1024^2 x 800 (5.4e10) 4824 / 2336; f16
+    // storage, whose half staging is faster here: 24 of 400^2 x 500 (1.9e9) 167 / 172, 32 (2.6e9)
+    // 240 / 185, 64 of 1024^2 x 800 3486 / 1625.
+    const double updates = (double) n_slices * roi_w * roi_h * P_in;
+    if (!fixed && !ctx->bp_slices && !ctx->bp_chunk && n_slices >= 12 &&
+        updates >= (dtype == UFOMI_F16 ? 2.5e9 : 1e9)) {
+        const ufomi_bp_stack st = {d_sino, dtype, W, P_in, n_slices, sino_pitch, trig, axis, (float) prm->roi_x,
+                                   (float) prm->roi_y, roi_w, roi_h, d_out, out_pitch};
+        int done = 0;
+        if ((rc = ufomi_bp_mfma(ctx, st, &done))) return rc;
+        if (done == n_slices) return UFOMI_OK;
+        n_slices -= done;
+        d_out += (size_t) done * out_pitch;
+        d_sino = (const char *) d_sino + (size_t) done * sino_pitch * (dtype == UFOMI_F32 ? 4 : 2);
+    }
+
     // Tile configuration: slices sharing a tile (S), angles per LDS chunk (A),
     // half-precision staging for f16 storage; ufomi_bp_configure overrides.
     // Measured on MI355X (2048 slices of 1800 x 2048): S = 8, A = 8 is the
@@ -819,6 +863,26 @@ extern "C" int ufomi_bp_parallel_noalloc(ufomi_ctx *ctx, const void *d_sino, int
         return ufomi_fail(UFOMI_ERR_ARG, "the preallocated scratch of device %d was not set up (ufomi_create)",
                           ctx->device);
     return bp_parallel_impl(ctx, d_sino, dtype, W, P_in, n_slices, sino_pitch, prm, d_out, out_pitch, +1, true, fixed);
+}
+
+int ufomi_bp_nonfinite(ufomi_ctx *ctx, const ufomi_bp_stack &st, int s0, int ns, int n64, int n32,
+                       const unsigned *maxbits)
+{
+    const int tiles_x = (st.roi_w + kTile - 1) / kTile, tiles = tiles_x * ((st.roi_h + kTile - 1) / kTile);
+    auto go = [&](auto *in) {
+        using InT = std::remove_const_t<std::remove_pointer_t<decltype(in)>>;
+        hipLaunchKernelGGL(bp_nonfinite_kernel<InT>, dim3(512), dim3(kThreads), 0, ctx->stream,
+                           in + (size_t) s0 * st.sino_pitch, (long) st.sino_pitch, st.W, st.P, st.trig, st.axis,
+                           st.roi_x, st.roi_y, st.roi_w, st.roi_h, ns, n64, n32, maxbits,
+                           st.out + (size_t) s0 * st.out_pitch, (long) st.out_pitch, tiles_x, tiles);
+        UFOMI_CHECK_LAUNCH();
+        return (int) UFOMI_OK;
+    };
+    switch (st.dtype) {
+    case UFOMI_F16: return go((const __half *) st.sino);
+    case UFOMI_BF16: return go((const __hip_bfloat16 *) st.sino);
+    default: return go((const float *) st.sino);
+    }
 }
 
 // ---- persistent batch kernel launchers

@@ -134,6 +134,12 @@ extern "C" int ufomi_destroy(ufomi_ctx *ctx)
         (void) hipFree(ctx->lut);
     if (ctx->bp_part)
         (void) hipFree(ctx->bp_part);
+    if (ctx->ws) {
+        (void) hipEventSynchronize(ctx->ws_event);  // its last use may be on an earlier stream
+        (void) hipFree(ctx->ws);
+    }
+    if (ctx->ws_event)
+        (void) hipEventDestroy(ctx->ws_event);
     if (ctx->scratch)
         (void) hipFree(ctx->scratch);
     if (ctx->hscratch)

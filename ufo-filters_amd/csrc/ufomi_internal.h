@@ -31,6 +31,12 @@ struct ufomi_ctx {
     // partial sums of angle-split backprojections of few tiles (grow-only)
     float *bp_part;
     size_t bp_part_bytes;
+    // row workspace of stack backprojections (bp_mfma.hip, grow-only), the event of its last
+    // use and the stream of that use
+    void *ws;
+    size_t ws_bytes;
+    hipEvent_t ws_event;
+    hipStream_t ws_stream;
 };
 
 #define UFOMI_FFT_MAX 16384  // twiddle table length
@@ -79,6 +85,24 @@ int ufomi_bp_trig(ufomi_ctx *ctx, double angle_offset, double step, unsigned off
 int ufomi_bp_parallel_ex(ufomi_ctx *ctx, const void *d_sino, int dtype, int W, int P_in, int n_slices,
                          size_t sino_pitch, const ufomi_bp_params *prm, float *d_out, size_t out_pitch, int sin_sign,
                          bool half_staging);
+
+// A stack of slices for the matrix-core backprojector (bp_mfma.hip), arguments checked.
+struct ufomi_bp_stack {
+    const void *sino;
+    int dtype, W, P, n_slices;
+    size_t sino_pitch;
+    const float2 *trig;
+    float axis, roi_x, roi_y;
+    int roi_w, roi_h;
+    float *out;
+    size_t out_pitch;
+};
+// Backprojects the first *done slices (0: none, the caller's other path takes all of them).
+int ufomi_bp_mfma(ufomi_ctx *ctx, const ufomi_bp_stack &st, int *done);
+// Slices s0 .. s0 + ns - 1 again where a unit that holds an Inf or a NaN (maxbits) was left out:
+// units of 64 slices up to n64, of 32 up to n32, of 16 after.
+int ufomi_bp_nonfinite(ufomi_ctx *ctx, const ufomi_bp_stack &st, int s0, int ns, int n64, int n32,
+                       const unsigned *maxbits);
 
 // Takes the calling thread's current device's address of the preallocated
 // scratch of ufomi_bp_parallel_noalloc (once per device; ufomi_create).

@@ -12,6 +12,8 @@
 // Both are elementwise and bound by HBM.
 #include "ufomi_internal.h"
 
+#include <algorithm>
+
 // Every float operation rounds on its own, as in the reference kernels' source
 // (hipcc would otherwise fuse a * b + c into one FMA).
 #pragma clang fp contract(off)
@@ -20,30 +22,75 @@ namespace {
 
 constexpr int kThreads = 256;
 
-__device__ __forceinline__ float ffc_one(float v, float dk, float fl, bool absorb, bool fix)
+// (data - d) / (f - d), or log((f - d) / (data - d)), with f - d given.
+__device__ __forceinline__ float ffc_one(float v, float dk, float range, bool absorb, bool fix)
 {
-    float r = absorb ? logf(((fl - dk) / (v - dk)))
-                     : ((v - dk) / (fl - dk));
+    float r = absorb ? logf((range / (v - dk)))
+                     : ((v - dk) / range);
     if (fix && (isnan(r) || isinf(r)))
         r = 0.0f;
     return r;
 }
 
+constexpr int kItems = 8;  // items per thread
+
+template <int V> struct Vec { float v[V]; };
+template <int V> __device__ __forceinline__ Vec<V> load_vec(const float *p)
+{
+    Vec<V> r;
+    if constexpr (V == 4) {
+        const float4 q = *(const float4 *) p;
+        r.v[0] = q.x; r.v[1] = q.y; r.v[2] = q.z; r.v[3] = q.w;
+    } else {
+        r.v[0] = *p;
+    }
+    return r;
+}
+
+// A thread corrects V adjacent pixels of kItems items.  Bound by HBM at 8 bytes per pixel: a pixel
+// per thread with its own 64-bit division and dark and flat reads ran at 2.5 TB/s (400 items of
+// 1024^2: 1.32 ms); here the dark and flat are read once per kItems items while they do not
+// change, and 8 16-byte loads are in flight per thread (0.65 ms, 5.1 TB/s).
+template <int V>
 __global__ __launch_bounds__(kThreads) void ffc_kernel(const float *__restrict__ data, const float *__restrict__ dark,
                                                        const float *__restrict__ flat, float *__restrict__ out,
                                                        long plane, int W, int n, int n_dark, int n_flat,
                                                        int sino_in, int absorb, int fix, float dark_scale,
                                                        float flat_scale)
 {
-    const long i = (long) blockIdx.x * kThreads + threadIdx.x;
-    if (i >= plane * n)
+    const long e = ((long) blockIdx.x * kThreads + threadIdx.x) * V;
+    if (e >= plane)
         return;
-    const long item = i / plane, e = i - item * plane;
-    const long ce = sino_in ? e % W : e;
+    const long ce = sino_in ? (long) ((unsigned long) e % (unsigned) W) : e;
     const long cplane = sino_in ? W : plane;
-    const float dk = dark[min(item, (long) n_dark - 1) * cplane + ce] * dark_scale;
-    const float fl = flat[min(item, (long) n_flat - 1) * cplane + ce] * flat_scale;
-    out[i] = ffc_one(data[i], dk, fl, absorb != 0, fix != 0);
+    const int i0 = blockIdx.y * kItems;
+    Vec<V> x[kItems];
+#pragma unroll
+    for (int k = 0; k < kItems; k++)
+        if (i0 + k < n) x[k] = load_vec<V>(data + (long) (i0 + k) * plane + e);
+    Vec<V> dk, range;
+#pragma unroll
+    for (int k = 0; k < kItems; k++) {
+        const int item = i0 + k;
+        if (item >= n) break;
+        if (k == 0 || item < n_dark || item < n_flat) {
+            dk = load_vec<V>(dark + min(item, n_dark - 1) * cplane + ce);
+            const Vec<V> fl = load_vec<V>(flat + min(item, n_flat - 1) * cplane + ce);
+#pragma unroll
+            for (int j = 0; j < V; j++) {
+                dk.v[j] = dk.v[j] * dark_scale;
+                range.v[j] = fl.v[j] * flat_scale - dk.v[j];
+            }
+        }
+        float r[V];
+#pragma unroll
+        for (int j = 0; j < V; j++) r[j] = ffc_one(x[k].v[j], dk.v[j], range.v[j], absorb != 0, fix != 0);
+        float *o = out + (long) item * plane + e;
+        if constexpr (V == 4)
+            *(float4 *) o = make_float4(r[0], r[1], r[2], r[3]);
+        else
+            o[0] = r[0];
+    }
 }
 
 __global__ __launch_bounds__(kThreads) void average_kernel(const float *__restrict__ in, long elems, int n,
@@ -72,13 +119,29 @@ extern "C" int ufomi_flat_field_correct(ufomi_ctx *ctx, const float *d_data, int
     if (!d_data || !d_dark || !d_flat || !d_out || W <= 0 || H <= 0 || n <= 0 || n_dark <= 0 || n_flat <= 0)
         return ufomi_fail(UFOMI_ERR_ARG, "invalid flat-field arguments");
     const long plane = (long) W * H, total = plane * n;
-    const long blocks = (total + kThreads - 1) / kThreads;
-    if (blocks >= (1L << 31))
+    if ((total + kThreads - 1) / kThreads >= (1L << 31))
         return ufomi_fail(UFOMI_ERR_ARG, "flat-field batch too large for one launch");
-    hipLaunchKernelGGL(ffc_kernel, dim3((unsigned) blocks), dim3(kThreads), 0, ctx->stream, d_data, d_dark, d_flat,
-                       d_out, plane, W, n, n_dark, n_flat, sinogram_input, absorption_correct, fix_nan_and_inf,
-                       dark_scale, flat_scale);
-    UFOMI_CHECK_LAUNCH();
+    // 16-byte accesses where every pixel group of an item (and of a dark or flat row) is aligned
+    const bool a16 = plane % 4 == 0 && (!sinogram_input || W % 4 == 0) &&
+                     (((uintptr_t) d_data | (uintptr_t) d_dark | (uintptr_t) d_flat | (uintptr_t) d_out) & 15) == 0;
+    const int per = kThreads * (a16 ? 4 : 1);
+    // the grid's second axis holds 65535 blocks: longer batches go in several launches
+    for (long first = 0; first < n; first += 65535L * kItems) {
+        const int count = (int) std::min<long>(n - first, 65535L * kItems);
+        const dim3 grid((unsigned) ((plane + per - 1) / per), (unsigned) ((count + kItems - 1) / kItems));
+        const long dplane = sinogram_input ? W : plane;
+        const float *dk = d_dark + std::min<long>(first, n_dark - 1) * dplane;
+        const float *fl = d_flat + std::min<long>(first, n_flat - 1) * dplane;
+        const int nd = (int) std::max<long>(1, n_dark - first), nf = (int) std::max<long>(1, n_flat - first);
+        auto go = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, grid, dim3(kThreads), 0, ctx->stream, d_data + first * plane, dk, fl,
+                               d_out + first * plane, plane, W, count, nd, nf, sinogram_input, absorption_correct,
+                               fix_nan_and_inf, dark_scale, flat_scale);
+        };
+        if (a16) go(ffc_kernel<4>);
+        else go(ffc_kernel<1>);
+        UFOMI_CHECK_LAUNCH();
+    }
     return UFOMI_OK;
 }
 

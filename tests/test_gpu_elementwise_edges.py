@@ -37,3 +37,19 @@ def test_flat_field_runs(ctx, torch_dev, n, h, w, shift, sino, nd, nf):
         ref = oracle.flat_field_correct_ref32(data[i:i + 1], dark[min(i, nd - 1)], flat[min(i, nf - 1)], True, False,
                                               False, 0.5, 1.5)[0]
         assert rel_l2(got[i], ref) < 1e-6, i  # one rounding of logf (2 ulp) over the oracle's
+
+
+@pytest.mark.parametrize("p,h,w,shift", [(1, 2, 4, 0), (4, 3, 260, 0), (5, 5, 62, 0), (9, 4, 8, 2), (6, 2, 7, 0)])
+@pytest.mark.parametrize("per_projection", [False, True])
+def test_cone_weight_runs(ctx, torch_dev, p, h, w, shift, per_projection):
+    rng = np.random.default_rng(p + w)
+    x = rng.uniform(0.5, 2.0, (p, h, w)).astype(np.float32)
+    cx = list(w / 2.0 + 0.25 * np.arange(p)) if per_projection else w / 2.0
+    sod = list(300.0 + np.arange(p)) if per_projection else 300.0
+    out = _dev(np.full((p, h, w), np.nan), torch_dev, shift)
+    ctx.cone_weight(_dev(x, torch_dev, shift), out, w, h, p, cx, h / 2.0, sod, 500.0, 0.0)
+    got = out.cpu().numpy()
+    for i in range(p):
+        ref = oracle.cone_weight_ref32(x[i], cx[i] if per_projection else cx, h / 2.0,
+                                       sod[i] if per_projection else sod, 500.0, 0.0)
+        np.testing.assert_allclose(got[i], ref, rtol=2e-6)

@@ -84,7 +84,7 @@ int enqueue(ufomi_fbp_batch *b, hipStream_t stream, int stages)
     int rc;
     if (stages & 1)
         for (const Group &g : b->groups)
-            if ((rc = ufomi_ramp_segments_launch(stream, b->ctx->twiddles, g.N, b->dtype, g.d_segs, g.nseg,
+            if ((rc = ufomi_ramp_segments_launch(stream, b->ctx->tw16, g.N, b->dtype, g.d_segs, g.nseg,
                                                  g.nblocks, g.d_coef, g.pair)))
                 return rc;
     if (stages & 2)

@@ -1,5 +1,6 @@
 // Context, errors, scratch memory and the host-side filter coefficients.
 #include "ufomi_internal.h"
+#include "fft16.h"
 
 #include <cmath>
 #include <cstdlib>
@@ -103,11 +104,30 @@ extern "C" int ufomi_create(int device, ufomi_ctx **out)
         double a = 2.0 * M_PI * (double) k / (double) M;
         tw[k] = make_float2((float) cos(a), (float) -sin(a));
     }
-    if (hipMalloc(&ctx->flags, 256) != hipSuccess || hipMalloc(&ctx->twiddles, M * sizeof(float2)) != hipSuccess ||
-        hipMemcpy(ctx->twiddles, tw.data(), M * sizeof(float2), hipMemcpyHostToDevice) != hipSuccess) {
+    // The register FFT's twiddle arrays, pass by pass for every size (fft16::Tab), behind them.
+    tw.resize(M + fft16::Tab::base(2 * UFOMI_FFT_MAX_N));
+    float2 *o = tw.data() + M;
+    auto emit = [&](int R, int Ns) {
+        const int step = M / (R * Ns);
+        for (int e = 0; e < R - 1; e++)
+            for (int k = 0; k < Ns; k++) {
+                const int q = (e - 3) / 3, r = (e - 3) % 3 + 1;
+                *o++ = tw[(R < 16 ? (e + 1) * k : e < 3 ? 4 * (e + 1) * k : r * (k + q * Ns)) * step];
+            }
+    };
+    for (int N = 16; N <= UFOMI_FFT_MAX_N; N *= 2) {
+        const int r0 = fft16::Tab::radix0(N);
+        for (int Ns = r0; Ns < N; Ns *= 16) emit(16, Ns);
+        if (r0 == 16) continue;
+        for (int Ns = 16; Ns < N / r0; Ns *= 16) emit(16, Ns);
+        emit(r0, N / r0);
+    }
+    if (hipMalloc(&ctx->flags, 256) != hipSuccess || hipMalloc(&ctx->twiddles, tw.size() * sizeof(float2)) != hipSuccess ||
+        hipMemcpy(ctx->twiddles, tw.data(), tw.size() * sizeof(float2), hipMemcpyHostToDevice) != hipSuccess) {
         free(ctx);
         return ufomi_fail(UFOMI_ERR_HIP, "twiddle table upload failed");
     }
+    ctx->tw16 = ctx->twiddles + M;
     if (int rc = ufomi_bp_noalloc_setup(device)) {
         (void) hipFree(ctx->flags);
         (void) hipFree(ctx->twiddles);
@@ -140,6 +160,9 @@ extern "C" int ufomi_destroy(ufomi_ctx *ctx)
     }
     if (ctx->ws_event)
         (void) hipEventDestroy(ctx->ws_event);
+    for (ufomi_chirp &c : ctx->chirps)
+        if (c.table)
+            (void) hipFree(c.table);
     if (ctx->scratch)
         (void) hipFree(ctx->scratch);
     if (ctx->hscratch)

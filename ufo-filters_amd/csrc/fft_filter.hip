@@ -8,7 +8,7 @@
 // N = 4, 8: a radix-4 Stockham FFT in LDS (lds_fft): TF = N/4 threads per
 // transform, each keeping its butterflies in registers between the read and
 // write halves of a pass.
-// Twiddles come from the context's FP64-accurate table (read through L2).
+// Twiddles come from the context's FP64-accurate tables (read through L2).
 #include "ufomi_internal.h"
 #include "fft16.h"
 
@@ -406,7 +406,7 @@ extern "C" int ufomi_fft_rows(ufomi_ctx *ctx, const float *d_in, int W, int P, i
             using PL = fft16::Plan<NN>;
             const unsigned blocks = (unsigned) (((long) P + PL::G - 1) / PL::G);
             hipLaunchKernelGGL(fft16_rows_kernel<NN>, dim3(blocks), dim3(kThreads), lds16_bytes<NN>(), ctx->stream,
-                               d_in, W, (long) P, (float2 *) d_out, ctx->twiddles);
+                               d_in, W, (long) P, (float2 *) d_out, ctx->tw16 + fft16::Tab::base(NN));
             UFOMI_CHECK_LAUNCH();
             return (int) UFOMI_OK;
         });
@@ -440,7 +440,7 @@ extern "C" int ufomi_ifft_rows(ufomi_ctx *ctx, const float *d_in, int N, int P, 
             using PL = fft16::Plan<NN>;
             const unsigned blocks = (unsigned) (((long) P + PL::G - 1) / PL::G);
             hipLaunchKernelGGL(ifft16_rows_kernel<NN>, dim3(blocks), dim3(kThreads), lds16_bytes<NN>(), ctx->stream,
-                               (const float2 *) d_in, (long) P, crop, d_out, scale, ctx->twiddles);
+                               (const float2 *) d_in, (long) P, crop, d_out, scale, ctx->tw16 + fft16::Tab::base(NN));
             UFOMI_CHECK_LAUNCH();
             return (int) UFOMI_OK;
         });
@@ -504,7 +504,8 @@ extern "C" int ufomi_ramp_filter(ufomi_ctx *ctx, const float *d_in, int W, int P
             using PL = fft16::Plan<NN>;
             const unsigned blocks = (unsigned) (((long) P + PL::G - 1) / PL::G);
             hipLaunchKernelGGL((ramp16_kernel<NN, OutT>), dim3(blocks), dim3(kThreads), lds16_bytes<NN>(),
-                               ctx->stream, d_in, W, (long) P, d_coef, d_flag, crop, out, scale, ctx->twiddles);
+                               ctx->stream, d_in, W, (long) P, d_coef, d_flag, crop, out, scale,
+                               ctx->tw16 + fft16::Tab::base(NN));
             UFOMI_CHECK_LAUNCH();
             return (int) UFOMI_OK;
         };
@@ -544,7 +545,7 @@ long ufomi_ramp_rows_per_block(int N, int pair)
     return g < 0 ? g : (long) g * (pair ? 2 : 1);
 }
 
-int ufomi_ramp_segments_launch(hipStream_t stream, const float2 *tw, int N, int out_dtype,
+int ufomi_ramp_segments_launch(hipStream_t stream, const float2 *tw16, int N, int out_dtype,
                                const ufomi_ramp_seg *d_segs, int nseg, long nblocks, const float *d_coef, int pair)
 {
     if (nblocks <= 0 || nblocks > 0x7fffffffL || nseg <= 0)
@@ -555,7 +556,8 @@ int ufomi_ramp_segments_launch(hipStream_t stream, const float2 *tw, int N, int 
         auto go = [&](auto *tag) {
             using OutT = std::remove_pointer_t<decltype(tag)>;
             hipLaunchKernelGGL((ramp16_segments_kernel<NN, OutT>), dim3((unsigned) nblocks), dim3(kThreads),
-                               lds16_bytes<NN>(), stream, d_segs, nseg, d_coef, pair, scale, tw);
+                               lds16_bytes<NN>(), stream, d_segs, nseg, d_coef, pair, scale,
+                               tw16 + fft16::Tab::base(NN));
             UFOMI_CHECK_LAUNCH();
             return (int) UFOMI_OK;
         };

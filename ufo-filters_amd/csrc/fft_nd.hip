@@ -4,24 +4,21 @@
 // src/ufo-ifft-task.c:111-306, src/common/ufo-fft.c:161-354).
 //
 // A transform is a sequence of axis passes.  One pass is one kernel launch
-// that moves every line of the array along one axis through LDS:
-//   load the line (zero beyond the input extent) -> FFT in LDS -> store
-// the first n_out outputs.  Sizes that are not a power of two (and powers of
-// two below 16) use Bluestein's algorithm (L. Bluestein, "A linear filtering
-// approach to the computation of the discrete Fourier transform", 1970)
-// fused into the same pass:
+// that moves every line of the array along one axis through the registers of
+// a workgroup (fft16.h): load the line (zero beyond the input extent) -> FFT
+// -> store the first n_out outputs.  Sizes that are not a power of two (and
+// powers of two below 16) use Bluestein's algorithm (L. Bluestein, "A linear
+// filtering approach to the computation of the discrete Fourier transform",
+// 1970) fused into the same pass:
 //   X_k = c_k * sum_n (x_n c_n) conj(c_{k-n}),   c_n = exp(dir i pi n^2 / M),
 // a circular convolution of length L >= 2M - 1 done as FFT_L, a product with
-// the precomputed spectrum of conj(c) (1/L folded in), and an inverse FFT_L,
-// all in LDS.  The reference runs the same mathematics as a chain of
-// separate kernels over global memory (spread, modulate, FFT, multiply,
-// IFFT, multiply, pack); here each axis costs one HBM round trip.
+// the precomputed spectrum of conj(c) (1/L folded in), and an inverse FFT_L.
+// The reference runs the same mathematics as a chain of separate kernels over
+// global memory (spread, modulate, FFT, multiply, IFFT, multiply, pack); here
+// each axis costs one HBM round trip.
 //
-// Lines along axis 0 are contiguous: a block takes G whole lines.  Lines
-// along axes 1 and 2 are strided: a block takes G neighbouring lines, so
-// one row of the block's tile is G consecutive complex values in memory
-// (coalesced), and LDS lines are padded by one element against bank
-// conflicts on the transposed write.
+// Axes longer than a pass holds run as the four-step split over
+// axis_dft_kernel, a radix-4 FFT in LDS.
 #include "ufomi_internal.h"
 #include "fft16.h"
 
@@ -53,10 +50,10 @@ struct Pass {
 __device__ __forceinline__ float2 load_as_complex(const float *p, long o) { return make_float2(p[o], 0.0f); }
 __device__ __forceinline__ float2 load_as_complex(const float2 *p, long o) { return p[o]; }
 
-template <int BB, int DIR, bool CHIRP, typename InT, bool OUT_REAL>
+// A pass of the four-step split: lines through LDS.  Lines along axis 0 are contiguous; of strided
+// lines a block takes G neighbouring ones, so that one row of its tile is G consecutive values.
+template <int BB, int DIR, typename InT, bool OUT_REAL>
 __global__ __launch_bounds__(kThreads) void axis_dft_kernel(const InT *__restrict__ in, void *__restrict__ out_, Pass g,
-                                                            const float2 *__restrict__ chirp,
-                                                            const float2 *__restrict__ kern,
                                                             const float2 *__restrict__ tw)
 {
     extern __shared__ float2 lds[];
@@ -80,24 +77,12 @@ __global__ __launch_bounds__(kThreads) void axis_dft_kernel(const InT *__restric
         const int a = a0 + gl;
         float2 v = make_float2(0.0f, 0.0f);
         const bool inside = g.flat_in ? (long) a * g.in_a + (long) i * g.in_e < g.flat_in : i < g.n_in;
-        if (a < g.A && inside) {
+        if (a < g.A && inside)
             v = load_as_complex(in, (long) a * g.in_a + (long) b * g.in_b + (long) i * g.in_e);
-            if (CHIRP)
-                v = cmul(v, chirp[i]);
-        }
         lds[gl * g.Ls + i] = v;
     }
     __syncthreads();
-    float2 *x = lds + f * g.Ls;
-    if (CHIRP) {
-        lds_fft<BB, -1>(x, g.L, g.log2L, t, TF, tw);
-        for (int i = t; i < g.L; i += TF)
-            x[i] = cmul(x[i], kern[i]);
-        __syncthreads();
-        lds_fft<BB, +1>(x, g.L, g.log2L, t, TF, tw);
-    } else {
-        lds_fft<BB, DIR>(x, g.L, g.log2L, t, TF, tw);
-    }
+    lds_fft<BB, DIR>(lds + f * g.Ls, g.L, g.log2L, t, TF, tw);
 
     const int total_out = g.G * g.n_out;
     for (int idx = threadIdx.x; idx < total_out; idx += kThreads) {
@@ -113,8 +98,6 @@ __global__ __launch_bounds__(kThreads) void axis_dft_kernel(const InT *__restric
         if (a >= g.A || (g.flat_out && (long) a * g.out_a + (long) i * g.out_e >= g.flat_out))
             continue;
         float2 y = lds[gl * g.Ls + i];
-        if (CHIRP)
-            y = cmul(y, chirp[i]);
         if (g.tw_n) {
             // (a i mod tw_n) / tw_n is exact in float for a power-of-two tw_n
             const long q = ((long) a * i) & (g.tw_n - 1);
@@ -123,6 +106,88 @@ __global__ __launch_bounds__(kThreads) void axis_dft_kernel(const InT *__restric
             y = cmul(y, make_float2(cs, DIR * sn));
         }
         const long o = (long) a * g.out_a + (long) b * g.out_b + (long) i * g.out_e;
+        if (OUT_REAL)
+            ((float *) out_)[o] = y.x * g.scale;
+        else
+            ((float2 *) out_)[o] = make_float2(y.x * g.scale, y.y * g.scale);
+    }
+}
+
+// A product that is rounded before the butterflies that follow (else the compiler fuses it into
+// their sums, and the result depends on which ones).
+__device__ __forceinline__ float2 rounded(float2 a)
+{
+    asm("" : "+v"(a.x), "+v"(a.y));
+    return a;
+}
+
+// One pass over lines of L points held in registers, P::G lines per workgroup, CHIRP for Bluestein
+// (DIR is then in the tables).  Neighbouring strided lines sit in neighbouring lanes; longer ones,
+// one per workgroup, touch 8 bytes of a cache line, so the blocks are dealt out such that the lines
+// sharing it run on one XCD and find it in that L2.  Bound by vector issue and the twiddle loads:
+// the passes of 12 transforms of 1500 x 1100 (L = 4096) take 0.22 ms (axis 0) and 0.39 ms (axis 1,
+// 8 bytes of a line each); with the lines in LDS and radix-4 passes they took 1.06-1.71 ms, to the
+// same bits (the twiddles and roundings are those of radix-4 passes).
+template <int L, int DIR, bool CHIRP, typename InT, bool OUT_REAL>
+__global__ __launch_bounds__(kThreads) void axis16_kernel(const InT *__restrict__ in, void *__restrict__ out_, Pass g,
+                                                          const float2 *__restrict__ chirp,
+                                                          const float2 *__restrict__ kern,
+                                                          const float2 *__restrict__ tw)
+{
+    using P = fft16::Plan<L>;
+    constexpr int R0 = P::radix(0), RL = P::radix(P::NPASS - 1);
+    constexpr int RO = CHIRP && R0 == RL ? R0 : RL;  // radix whose slots hold the outputs
+    extern __shared__ float2 lds[];
+    const bool strided = g.in_e != 1;
+    const int f = strided ? threadIdx.x % P::G : threadIdx.x / P::TF;
+    const int t = strided ? threadIdx.x / P::G : threadIdx.x % P::TF;
+    float2 *x = lds + (size_t) f * fft16::Lds<L>::STRIDE;
+    const unsigned nb = gridDim.x, q8 = nb >> 3;
+    const unsigned blk = blockIdx.x < (q8 << 3) ? (blockIdx.x & 7) * q8 + (blockIdx.x >> 3) : blockIdx.x;
+    const unsigned ablocks = (unsigned) (g.A + P::G - 1) / P::G;
+    const unsigned b = blk / ablocks;
+    const int a = (int) (blk - b * ablocks) * P::G + f;
+    const bool valid = a < g.A;
+
+    const InT *src = in + (long) (valid ? a : 0) * g.in_a + (long) b * g.in_b + (long) t * g.in_e;
+    float2 v[P::V];
+#pragma unroll
+    for (int s = 0; s < P::V; s++) {
+        const int k = fft16::slot_index<L, R0>(0, s);
+        v[s] = valid && t + k < g.n_in ? load_as_complex(src, (long) k * g.in_e) : make_float2(0.0f, 0.0f);
+    }
+    if constexpr (CHIRP) {
+#pragma unroll
+        for (int s = 0; s < P::V; s++) {
+            const int e = fft16::slot_index<L, R0>(t, s);
+            if (e < g.n_in) v[s] = rounded(fft16::cmul_v<false>(v[s], chirp[e]));
+        }
+        fft16::transform_forward_order<L, -1, true>(v, x, t, tw);
+#pragma unroll
+        for (int s = 0; s < P::V; s++) v[s] = rounded(fft16::cmul_v<false>(v[s], kern[fft16::slot_index<L, RL>(t, s)]));
+        if constexpr (R0 == RL) {
+            fft16::transform_reverse_order<L, +1, true>(v, x, t, tw);
+        } else {
+            // the inverse takes the passes in the same order: natural order through LDS
+            __syncthreads();
+#pragma unroll
+            for (int s = 0; s < P::V; s++) x[fft16::Lds<L>::at(fft16::slot_index<L, RL>(t, s))] = v[s];
+            __syncthreads();
+#pragma unroll
+            for (int s = 0; s < P::V; s++) v[s] = x[fft16::Lds<L>::at(fft16::slot_index<L, R0>(t, s))];
+            fft16::transform_forward_order<L, +1, true>(v, x, t, tw);
+        }
+    } else {
+        fft16::transform_forward_order<L, DIR, true>(v, x, t, tw);
+    }
+    const long o0 = (long) a * g.out_a + (long) b * g.out_b + (long) t * g.out_e;
+#pragma unroll
+    for (int s = 0; s < P::V; s++) {
+        const int k = fft16::slot_index<L, RO>(0, s);
+        if (!valid || t + k >= g.n_out) continue;
+        float2 y = v[s];
+        if constexpr (CHIRP) y = fft16::cmul_v<false>(y, chirp[t + k]);
+        const long o = o0 + (long) k * g.out_e;
         if (OUT_REAL)
             ((float *) out_)[o] = y.x * g.scale;
         else
@@ -191,10 +256,10 @@ void bluestein_tables(int M, int L, int dir, float2 *chirp, float2 *kern)
 
 struct PassSpec {
     Pass g;
-    int BB;
+    int BB;              // four-step split only
     bool chirp;
     int M;
-    size_t table_off;  // float2 offset of this pass's chirp table in the table block (kern follows)
+    const float2 *tables;  // chirp[M], then the kernel spectrum
 };
 
 // Lines along `axis` of a source array with extents S (x fastest) into a
@@ -213,9 +278,9 @@ int make_pass(int axis, const int S[3], const int D[3], const int E[3], int n_in
     ps->M = M;
     g.L = L;
     g.log2L = ufomi_log2(L);
-    ps->BB = L >= 8192 ? 8 : std::min(4, L / 16);
-    g.G = 1024 * ps->BB / L;
-    g.Ls = g.G > 1 ? L + 1 : L;
+    ps->tables = nullptr;
+    g.G = L >= 8192 ? 1 : 4096 / L;  // fft16::Plan's lines per workgroup
+    g.Ls = 0;
     g.n_in = n_in;
     g.n_out = n_out;
     g.scale = 1.0f;
@@ -246,9 +311,8 @@ int make_pass(int axis, const int S[3], const int D[3], const int E[3], int n_in
     return UFOMI_OK;
 }
 
-template <int DIR, bool CHIRP, typename InT, bool OUT_REAL>
-int launch_bb(hipStream_t s, const PassSpec &ps, const void *in, void *out, const float2 *chirp, const float2 *kern,
-              const float2 *tw)
+template <int DIR, typename InT, bool OUT_REAL>
+int launch_bb(hipStream_t s, const PassSpec &ps, const void *in, void *out, const float2 *tw)
 {
     const Pass &g = ps.g;
     const unsigned blocks = (unsigned) ((long) g.Bn * ((g.A + g.G - 1) / g.G));
@@ -256,8 +320,8 @@ int launch_bb(hipStream_t s, const PassSpec &ps, const void *in, void *out, cons
     switch (ps.BB) {
 #define UFOMI_AXIS_CASE(BBV)                                                                                       \
     case BBV:                                                                                                      \
-        hipLaunchKernelGGL((axis_dft_kernel<BBV, DIR, CHIRP, InT, OUT_REAL>), dim3(blocks), dim3(kThreads), lds, s, \
-                           (const InT *) in, out, g, chirp, kern, tw);                                             \
+        hipLaunchKernelGGL((axis_dft_kernel<BBV, DIR, InT, OUT_REAL>), dim3(blocks), dim3(kThreads), lds, s,       \
+                           (const InT *) in, out, g, tw);                                                          \
         break;
         UFOMI_AXIS_CASE(1)
         UFOMI_AXIS_CASE(2)
@@ -271,38 +335,83 @@ int launch_bb(hipStream_t s, const PassSpec &ps, const void *in, void *out, cons
 }
 
 template <int DIR, typename InT, bool OUT_REAL>
-int launch_pass(hipStream_t s, const PassSpec &ps, const void *in, void *out, const float2 *tables, const float2 *tw)
+int launch_pass(hipStream_t s, const PassSpec &ps, const void *in, void *out, const float2 *tw16)
 {
-    const float2 *chirp = tables + ps.table_off, *kern = chirp + ps.M;
-    return ps.chirp ? launch_bb<DIR, true, InT, OUT_REAL>(s, ps, in, out, chirp, kern, tw)
-                    : launch_bb<DIR, false, InT, OUT_REAL>(s, ps, in, out, nullptr, nullptr, tw);
+    const Pass &g = ps.g;
+    const unsigned blocks = (unsigned) ((long) g.Bn * ((g.A + g.G - 1) / g.G));
+    const float2 *chirp = ps.tables, *kern = chirp + ps.M, *tw = tw16 + fft16::Tab::base(g.L);
+    switch (g.L) {
+#define UFOMI_AXIS_CASE(LV)                                                                                          \
+    case LV: {                                                                                                       \
+        using P = fft16::Plan<LV>;                                                                                   \
+        const size_t lds = P::NPASS > 1 ? (size_t) P::G * fft16::Lds<LV>::STRIDE * sizeof(float2) : 0;               \
+        if (ps.chirp)                                                                                                \
+            hipLaunchKernelGGL((axis16_kernel<LV, 0, true, InT, OUT_REAL>), dim3(blocks), dim3(kThreads), lds, s,    \
+                               (const InT *) in, out, g, chirp, kern, tw);                                           \
+        else                                                                                                         \
+            hipLaunchKernelGGL((axis16_kernel<LV, DIR, false, InT, OUT_REAL>), dim3(blocks), dim3(kThreads), lds, s, \
+                               (const InT *) in, out, g, chirp, kern, tw);                                           \
+        break;                                                                                                       \
+    }
+        UFOMI_AXIS_CASE(16)
+        UFOMI_AXIS_CASE(32)
+        UFOMI_AXIS_CASE(64)
+        UFOMI_AXIS_CASE(128)
+        UFOMI_AXIS_CASE(256)
+        UFOMI_AXIS_CASE(512)
+        UFOMI_AXIS_CASE(1024)
+        UFOMI_AXIS_CASE(2048)
+        UFOMI_AXIS_CASE(4096)
+        UFOMI_AXIS_CASE(8192)
+#undef UFOMI_AXIS_CASE
+    default: return ufomi_fail(UFOMI_ERR_ARG, "internal: no axis kernel for %d points", g.L);
+    }
+    UFOMI_CHECK_LAUNCH();
+    return UFOMI_OK;
 }
 
-// Scratch: two complex intermediates of `tmp_elems` and the Bluestein tables of every pass.
-int setup_scratch(ufomi_ctx *ctx, PassSpec *ps, int np, int dir, size_t tmp_elems, float2 **tmp0, float2 **tmp1,
-                  float2 **tables)
+// The Bluestein tables of M points, from the context's few last used ones: they depend on the size
+// and direction alone, and forming them takes the host about a millisecond at 2048 points.
+int chirp_tables(ufomi_ctx *ctx, int M, int L, int dir, const float2 **out)
 {
-    size_t n_tab = 0;
-    for (int p = 0; p < np; p++) {
-        ps[p].table_off = n_tab;
-        if (ps[p].chirp)
-            n_tab += (size_t) ps[p].M + ps[p].g.L;
+    ufomi_chirp *slot = &ctx->chirps[0];
+    for (ufomi_chirp &c : ctx->chirps) {
+        if (c.table && c.M == M && c.dir == dir) {
+            c.used = ++ctx->chirp_clock;
+            *out = c.table;
+            return UFOMI_OK;
+        }
+        if (c.used < slot->used) slot = &c;
     }
+    std::vector<float2> h((size_t) M + L);
+    bluestein_tables(M, L, dir, h.data(), h.data() + M);
+    if (slot->table) {
+        UFOMI_HIP(hipDeviceSynchronize());  // earlier transforms, on any stream, may still read it
+        UFOMI_HIP(hipFree(slot->table));
+        *slot = ufomi_chirp{};
+    }
+    float2 *t = nullptr;
+    UFOMI_HIP(hipMalloc(&t, h.size() * sizeof(float2)));
+    if (hipMemcpy(t, h.data(), h.size() * sizeof(float2), hipMemcpyHostToDevice) != hipSuccess) {
+        (void) hipFree(t);
+        return ufomi_fail(UFOMI_ERR_HIP, "chirp table upload failed");
+    }
+    *slot = ufomi_chirp{t, M, dir, ++ctx->chirp_clock};
+    *out = t;
+    return UFOMI_OK;
+}
+
+// Scratch: two complex intermediates of `tmp_elems`; and the Bluestein tables of every pass.
+int setup_scratch(ufomi_ctx *ctx, PassSpec *ps, int np, int dir, size_t tmp_elems, float2 **tmp0, float2 **tmp1)
+{
     const size_t tmp_bytes = ((tmp_elems * sizeof(float2) + 255) / 256) * 256;
     void *base = nullptr;
-    int rc = ufomi_scratch(ctx, 2 * tmp_bytes + n_tab * sizeof(float2) + 256, &base);
+    int rc = ufomi_scratch(ctx, 2 * tmp_bytes, &base);
     if (rc) return rc;
     *tmp0 = (float2 *) base;
     *tmp1 = (float2 *) ((char *) base + tmp_bytes);
-    *tables = (float2 *) ((char *) base + 2 * tmp_bytes);
-    if (n_tab) {
-        std::vector<float2> h(n_tab);
-        for (int p = 0; p < np; p++)
-            if (ps[p].chirp)
-                bluestein_tables(ps[p].M, ps[p].g.L, dir, h.data() + ps[p].table_off,
-                                 h.data() + ps[p].table_off + ps[p].M);
-        if ((rc = ufomi_upload(ctx, *tables, h.data(), n_tab * sizeof(float2)))) return rc;
-    }
+    for (int p = 0; p < np; p++)
+        if (ps[p].chirp && (rc = chirp_tables(ctx, ps[p].M, ps[p].g.L, dir, &ps[p].tables))) return rc;
     return UFOMI_OK;
 }
 
@@ -361,9 +470,9 @@ int split_passes(ufomi_ctx *ctx, const void *in, long in_pitch, long valid, int 
         if (blocks <= 0 || blocks >= (1L << 31))
             return ufomi_fail(UFOMI_ERR_ARG, "transform of %d rows does not fit one launch", rows);
     }
-    int rc = launch_bb<DIR, false, InT, false>(ctx->stream, p1, in, tmp, nullptr, nullptr, ctx->twiddles);
+    int rc = launch_bb<DIR, InT, false>(ctx->stream, p1, in, tmp, ctx->twiddles);
     if (rc) return rc;
-    return launch_bb<DIR, false, float2, OUT_REAL>(ctx->stream, p2, tmp, out, nullptr, nullptr, ctx->twiddles);
+    return launch_bb<DIR, float2, OUT_REAL>(ctx->stream, p2, tmp, out, ctx->twiddles);
 }
 
 template <int DIR, typename InT, bool OUT_REAL>
@@ -624,14 +733,14 @@ int axis_by_axis(ufomi_ctx *ctx, const float *d_in, bool in_complex, const int n
             PassSpec ps;
             if ((rc = make_pass(a, Ss[p], Ds[p], Es[p], nin[p], nout[p], m[a], &ps))) break;
             ps.g.scale = scale;
-            float2 *t0, *t1, *tables;
-            if ((rc = setup_scratch(ctx, &ps, 1, DIR, 1, &t0, &t1, &tables))) break;
+            float2 *t0, *t1;
+            if ((rc = setup_scratch(ctx, &ps, 1, DIR, 1, &t0, &t1))) break;
             if (real_in)
-                rc = launch_pass<DIR, float, false>(ctx->stream, ps, src, dst, tables, ctx->twiddles);
+                rc = launch_pass<DIR, float, false>(ctx->stream, ps, src, dst, ctx->tw16);
             else if (real_out)
-                rc = launch_pass<DIR, float2, true>(ctx->stream, ps, src, dst, tables, ctx->twiddles);
+                rc = launch_pass<DIR, float2, true>(ctx->stream, ps, src, dst, ctx->tw16);
             else
-                rc = launch_pass<DIR, float2, false>(ctx->stream, ps, src, dst, tables, ctx->twiddles);
+                rc = launch_pass<DIR, float2, false>(ctx->stream, ps, src, dst, ctx->tw16);
         } else if (real_in) {
             rc = long_axis<DIR, float, false>(ctx, a, src, Ss[p], Ds[p], Es[p], nin[p], m[a], nout[p], scale, dst);
         } else if (real_out) {
@@ -702,8 +811,8 @@ extern "C" int ufomi_fft_nd(ufomi_ctx *ctx, const float *d_in, int in_complex, c
             tmp_elems = std::max(tmp_elems, (size_t) D[0] * D[1] * D[2]);
         S[a] = m[a];
     }
-    float2 *tmp[2], *tables;
-    if ((rc = setup_scratch(ctx, ps, dimensions, -1, tmp_elems, &tmp[0], &tmp[1], &tables))) return rc;
+    float2 *tmp[2];
+    if ((rc = setup_scratch(ctx, ps, dimensions, -1, tmp_elems, &tmp[0], &tmp[1]))) return rc;
     bool padded_batch = false;
     for (int k = dimensions; k < 3; k++)
         padded_batch |= m[k] > n[k];
@@ -713,9 +822,9 @@ extern "C" int ufomi_fft_nd(ufomi_ctx *ctx, const float *d_in, int in_complex, c
     for (int a = 0; a < dimensions; a++) {
         void *dst = a == dimensions - 1 ? (void *) d_out : (void *) tmp[a & 1];
         if (a == 0 && !in_complex)
-            rc = launch_pass<-1, float, false>(ctx->stream, ps[a], src, dst, tables, ctx->twiddles);
+            rc = launch_pass<-1, float, false>(ctx->stream, ps[a], src, dst, ctx->tw16);
         else
-            rc = launch_pass<-1, float2, false>(ctx->stream, ps[a], src, dst, tables, ctx->twiddles);
+            rc = launch_pass<-1, float2, false>(ctx->stream, ps[a], src, dst, ctx->tw16);
         if (rc) return rc;
         src = dst;
     }
@@ -769,14 +878,14 @@ extern "C" int ufomi_ifft_nd(ufomi_ctx *ctx, const float *d_in, const int *m, in
             S[k] = D[k];
     }
     ps[np - 1].g.scale = (float) (1.0 / norm);
-    float2 *tmp[2], *tables;
-    if ((rc = setup_scratch(ctx, ps, np, +1, tmp_elems, &tmp[0], &tmp[1], &tables))) return rc;
+    float2 *tmp[2];
+    if ((rc = setup_scratch(ctx, ps, np, +1, tmp_elems, &tmp[0], &tmp[1]))) return rc;
     const void *src = d_in;
     for (int p = 0; p < np; p++) {
         if (p == np - 1) {
-            rc = launch_pass<+1, float2, true>(ctx->stream, ps[p], src, d_out, tables, ctx->twiddles);
+            rc = launch_pass<+1, float2, true>(ctx->stream, ps[p], src, d_out, ctx->tw16);
         } else {
-            rc = launch_pass<+1, float2, false>(ctx->stream, ps[p], src, tmp[p & 1], tables, ctx->twiddles);
+            rc = launch_pass<+1, float2, false>(ctx->stream, ps[p], src, tmp[p & 1], ctx->tw16);
             src = tmp[p & 1];
         }
         if (rc) return rc;

@@ -11,10 +11,18 @@
 
 #include "ufomi.h"
 
+// Bluestein tables of one transform size and direction (fft_nd.hip): chirp[M], kernel spectrum[L].
+struct ufomi_chirp {
+    float2 *table;
+    int M, dir;
+    unsigned long used;
+};
+
 struct ufomi_ctx {
     int device;
     hipStream_t stream;
     float2 *twiddles;        // exp(-2 pi i k / UFOMI_FFT_MAX), k < UFOMI_FFT_MAX
+    float2 *tw16;            // the same values laid out for the passes of every size (fft16::Tab)
     int *flags;              // small device words written by classification kernels
     void *scratch;           // grow-only device scratch
     size_t scratch_bytes;
@@ -37,6 +45,8 @@ struct ufomi_ctx {
     size_t ws_bytes;
     hipEvent_t ws_event;
     hipStream_t ws_stream;
+    ufomi_chirp chirps[8];   // the last used Bluestein tables (at most 96 KiB each)
+    unsigned long chirp_clock;
 };
 
 #define UFOMI_FFT_MAX 16384  // twiddle table length
@@ -124,7 +134,7 @@ struct ufomi_ramp_seg {
 // Rows covered by one block of the radix-16 ramp kernel for transform size N
 // (2 G when `pair`); < 0 (with the error set) when N has no such kernel.
 long ufomi_ramp_rows_per_block(int N, int pair);
-int ufomi_ramp_segments_launch(hipStream_t stream, const float2 *tw, int N, int out_dtype,
+int ufomi_ramp_segments_launch(hipStream_t stream, const float2 *tw16, int N, int out_dtype,
                                const ufomi_ramp_seg *d_segs, int nseg, long nblocks, const float *d_coef, int pair);
 
 // One single-slice request of a persistent backprojection launch.

@@ -1,0 +1,78 @@
+"""Pipelines whose stage batches are blocks the context keeps and whose last stage writes the
+caller's memory: the results are those of the single calls for every kind of destination, and
+batches of changing sizes and streams do not disturb each other."""
+import ctypes
+
+import pytest
+
+torch = pytest.importorskip("torch")
+import ufo_tasks  # noqa: E402
+import ufomi  # noqa: E402
+
+pytestmark = pytest.mark.gpu
+CHAIN = "fft dimensions=1 size-x=%d ! filter ! ifft dimensions=1 crop-width=%d"
+
+
+def _text(W, last):
+    N = 1 << (2 * W - 1).bit_length()
+    chain = CHAIN % (N, W)
+    return chain + {"ifft": "", "backproject": " ! backproject axis-pos=%r" % (W / 2.0),
+                    "average": " ! average", "transpose": " ! transpose-projections number=7"}[last]
+
+
+def _run(ctx, text, x, out_ptr, cap, req_hw=None):
+    pl = ufo_tasks.Pipeline(text)
+    req, oreq, err, n = ufo_tasks.Requisition(), ufo_tasks.Requisition(), ufo_tasks.Error(), ctypes.c_int()
+    req.n_dims = 2
+    req.dims[0], req.dims[1], req.dims[2] = x.shape[2], x.shape[1], 1
+    rc = pl.L.ufomi_pipeline_run(pl.h, ctx.h, x.data_ptr(), ctypes.byref(req), x.shape[0], out_ptr, cap,
+                                 ctypes.byref(n), ctypes.byref(oreq), ctypes.byref(err))
+    elems = n.value * oreq.dims[0] * oreq.dims[1]
+    return rc, elems
+
+
+@pytest.mark.parametrize("last", ["ifft", "backproject", "average", "transpose"])
+def test_destinations_agree(last):
+    W, P, S = 65, 9, 5
+    ctx = ufomi.Context(0, torch.cuda.current_stream())
+    x = torch.randn(S, P, W, device="cuda")
+    text = _text(W, last)
+    cap = 4 * 9 * 7 * 65 * 65
+    plain = torch.full((cap // 4 + 64,), 7.0, device="cuda")
+    rc, n = _run(ctx, text, x, plain.data_ptr() + 4, cap)       # not aligned: the result is copied
+    assert rc == 0 and n > 0 and plain[0] == 7.0 and bool((plain[1 + n:] == 7.0).all())
+    want = plain[1:1 + n].clone()
+    direct = torch.full((cap // 4,), 7.0, device="cuda")
+    rc, m = _run(ctx, text, x, direct.data_ptr(), 4 * n)        # exactly large enough
+    assert rc == 0 and m == n
+    assert torch.equal(direct[:n], want) and bool((direct[n:] == 7.0).all())
+    direct.fill_(7.0)
+    rc, _ = _run(ctx, text, x, direct.data_ptr(), 4 * n - 4)    # too small: refused, nothing written
+    assert rc != 0 and bool((direct == 7.0).all())
+    host = torch.zeros(n, pin_memory=True)                      # not device memory
+    rc, _ = _run(ctx, text, x, host.data_ptr(), 4 * n)
+    assert rc == 0 and torch.equal(host, want.cpu())
+    both = torch.zeros(max(n, x.numel()), device="cuda")        # the input's own memory
+    both[:x.numel()] = x.flatten()
+    rc, _ = _run(ctx, text, both[:x.numel()].view_as(x), both.data_ptr(), 4 * n)
+    assert rc == 0 and torch.equal(both[:n], want)
+
+
+def test_blocks_over_sizes_and_streams():
+    """Batches that grow, shrink and exceed what the context keeps, on two streams in turn."""
+    a, b = torch.cuda.Stream(), torch.cuda.Stream()
+    ctx, fresh = ufomi.Context(0, a), None
+    for i, (S, P, W) in enumerate([(1, 8, 32), (6, 40, 200), (1, 8, 32), (3, 700, 2048), (40, 900, 2048),
+                                   (6, 40, 200), (2, 700, 2048), (1, 1, 1)]):
+        st = (a, b)[i % 2]
+        ctx.set_stream(st)
+        with torch.cuda.stream(st):
+            x = torch.randn(S, P, W, device="cuda")
+            st.synchronize()
+            text = _text(W, "ifft") + " ! fft dimensions=1 ! ifft dimensions=1 crop-width=%d" % W if W > 1 else "average"
+            got, n, shape = ufo_tasks.Pipeline(text).run(ctx, x, out_bytes=4 * x.numel())
+            fresh = ufomi.Context(0, st)
+            ref, m, _ = ufo_tasks.Pipeline(text).run(fresh, x, out_bytes=4 * x.numel())
+            st.synchronize()
+            k = 4 * n * shape[0] * shape[1] if len(shape) == 2 else 4 * n
+            assert n == m and torch.equal(got[:k], ref[:k])

@@ -285,7 +285,7 @@ extern "C" int ufomi_fbp_batch_create(ufomi_ctx *ctx, const ufomi_fbp_request *r
         mix((uint64_t) W); mix((uint64_t) P); mix((uint64_t) N); mix((uint64_t) roi_w); mix((uint64_t) roi_h);
     }
 
-    hipError_t e = hipMalloc(&b->d_filtered, b->filtered_bytes);
+    hipError_t e = ufomi_malloc(ctx, (void **) &b->d_filtered, b->filtered_bytes);
     if (e != hipSuccess) {
         free_batch(b);
         return ufomi_fail(UFOMI_ERR_MEMORY, "cannot allocate %zu bytes of filtered rows: %s", b->filtered_bytes,

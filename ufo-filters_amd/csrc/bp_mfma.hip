@@ -457,7 +457,7 @@ int acquire_workspace(ufomi_ctx *ctx, size_t bytes)
             ctx->ws = nullptr;
             ctx->ws_bytes = 0;
         }
-        if (hipMalloc(&ctx->ws, bytes) != hipSuccess) {
+        if (ufomi_malloc(ctx, &ctx->ws, bytes) != hipSuccess) {
             (void) hipGetLastError();  // the caller has a path without it
             ctx->ws = nullptr;
             return UFOMI_ERR_MEMORY;

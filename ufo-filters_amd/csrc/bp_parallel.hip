@@ -778,7 +778,7 @@ int bp_parallel_impl(ufomi_ctx *ctx, const void *d_sino, int dtype, int W, int P
                 ctx->bp_part = nullptr;
                 ctx->bp_part_bytes = 0;
             }
-            UFOMI_HIP(hipMalloc(&ctx->bp_part, bytes));
+            UFOMI_HIP(ufomi_malloc(ctx, (void **) &ctx->bp_part, bytes));
             ctx->bp_part_bytes = bytes;
         }
         part = ctx->bp_part;

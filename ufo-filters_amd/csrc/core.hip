@@ -5,6 +5,7 @@
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
+#include <mutex>
 #include <vector>
 
 static thread_local char g_error[512] = "";
@@ -39,6 +40,31 @@ int ufomi_enter(ufomi_ctx *ctx)
     return UFOMI_OK;
 }
 
+// Tasks give their blocks back wherever their last reference goes, also on another thread than
+// the context's.
+static std::mutex blocks_lock;
+
+static void trim_blocks(ufomi_ctx *ctx)
+{
+    std::lock_guard<std::mutex> guard(blocks_lock);
+    for (ufomi_block &b : ctx->blocks)
+        if (b.ptr && !b.busy) {
+            (void) hipFree(b.ptr);
+            b = {};
+        }
+}
+
+hipError_t ufomi_malloc(ufomi_ctx *ctx, void **ptr, size_t bytes)
+{
+    hipError_t e = hipMalloc(ptr, bytes);
+    if (e == hipErrorOutOfMemory) {
+        (void) hipGetLastError();
+        trim_blocks(ctx);
+        e = hipMalloc(ptr, bytes);
+    }
+    return e;
+}
+
 int ufomi_scratch(ufomi_ctx *ctx, size_t bytes, void **ptr)
 {
     if (bytes > ctx->scratch_bytes) {
@@ -49,7 +75,7 @@ int ufomi_scratch(ufomi_ctx *ctx, size_t bytes, void **ptr)
             ctx->scratch_bytes = 0;
         }
         size_t want = bytes < (1u << 20) ? (1u << 20) : bytes;
-        UFOMI_HIP(hipMalloc(&ctx->scratch, want));
+        UFOMI_HIP(ufomi_malloc(ctx, &ctx->scratch, want));
         ctx->scratch_bytes = want;
     }
     *ptr = ctx->scratch;
@@ -163,6 +189,7 @@ extern "C" int ufomi_destroy(ufomi_ctx *ctx)
     for (ufomi_chirp &c : ctx->chirps)
         if (c.table)
             (void) hipFree(c.table);
+    trim_blocks(ctx);
     if (ctx->scratch)
         (void) hipFree(ctx->scratch);
     if (ctx->hscratch)
@@ -186,7 +213,7 @@ extern "C" int ufomi_device_alloc(ufomi_ctx *ctx, size_t bytes, void **out)
     if (!out)
         return ufomi_fail(UFOMI_ERR_ARG, "null output pointer");
     *out = nullptr;
-    const hipError_t e = hipMalloc(out, bytes ? bytes : 1);
+    const hipError_t e = ufomi_malloc(ctx, out, bytes ? bytes : 1);
     if (e != hipSuccess) {
         (void) hipGetLastError();
         *out = nullptr;
@@ -207,6 +234,86 @@ extern "C" int ufomi_device_free(ufomi_ctx *ctx, void *ptr)
         UFOMI_HIP(hipFree(ptr));
     }
     return UFOMI_OK;
+}
+
+// Memory of the batches between the stages of a pipeline.  hipMalloc and hipFree of two buffers
+// of 79 MB cost 0.54 ms of a 2.1 ms run (FBP of 24 slices of 1024^2, 800 angles), so the context
+// keeps up to 8 blocks, 512 MiB in all; what does not fit is allocated and freed as it comes.  A
+// block becomes idle only after the context's stream has finished with it, so the next user may
+// be on any stream.  A block serves requests down to half its size.
+static const size_t kBlockBytes = (size_t) 512 << 20;
+
+extern "C" int ufomi_block_alloc(ufomi_ctx *ctx, size_t bytes, void **out)
+{
+    int rc = ufomi_enter(ctx);
+    if (rc) return rc;
+    {
+        std::lock_guard<std::mutex> guard(blocks_lock);
+        ufomi_block *best = nullptr;
+        size_t held = bytes;
+        int empty = 0;
+        for (ufomi_block &b : ctx->blocks) {
+            held += b.bytes;
+            empty += !b.ptr;
+            if (b.ptr && !b.busy && b.bytes >= bytes && b.bytes / 2 <= bytes && (!best || b.bytes < best->bytes))
+                best = &b;
+        }
+        if (best) {
+            best->busy = 1;
+            *out = best->ptr;
+            return UFOMI_OK;
+        }
+        // idle blocks of other sizes make room for this one
+        for (ufomi_block &b : ctx->blocks)
+            if (b.ptr && !b.busy && bytes <= kBlockBytes && (!empty || held > kBlockBytes)) {
+                held -= b.bytes;
+                empty++;
+                (void) hipFree(b.ptr);
+                b = {};
+            }
+    }
+    if ((rc = ufomi_device_alloc(ctx, bytes, out)))
+        return rc;
+    std::lock_guard<std::mutex> guard(blocks_lock);
+    ufomi_block *empty = nullptr;
+    size_t held = bytes;
+    for (ufomi_block &b : ctx->blocks) {
+        held += b.bytes;
+        if (!b.ptr) empty = &b;
+    }
+    if (empty && held <= kBlockBytes) *empty = {*out, bytes, 1};
+    return UFOMI_OK;
+}
+
+extern "C" int ufomi_block_free(ufomi_ctx *ctx, void *ptr)
+{
+    int rc = ufomi_enter(ctx);
+    if (rc || !ptr) return rc;
+    UFOMI_HIP(hipStreamSynchronize(ctx->stream));
+    {
+        std::lock_guard<std::mutex> guard(blocks_lock);
+        for (ufomi_block &b : ctx->blocks)
+            if (b.ptr == ptr) {
+                b.busy = 0;
+                return UFOMI_OK;
+            }
+    }
+    UFOMI_HIP(hipFree(ptr));
+    return UFOMI_OK;
+}
+
+// 1 when kernels on the context's device may write [ptr, ptr + bytes) directly with the widest
+// stores: aligned device memory of that device (not host or managed memory).
+extern "C" int ufomi_device_writable(ufomi_ctx *ctx, const void *ptr, size_t bytes)
+{
+    hipPointerAttribute_t a;
+    if ((uintptr_t) ptr % 256 || ufomi_enter(ctx))
+        return 0;
+    if (hipPointerGetAttributes(&a, ptr) != hipSuccess) {
+        (void) hipGetLastError();
+        return 0;
+    }
+    return a.type == hipMemoryTypeDevice && a.device == ctx->device && !a.isManaged;
 }
 
 extern "C" int ufomi_memcpy(ufomi_ctx *ctx, void *dst, const void *src, size_t bytes, int kind)

@@ -18,6 +18,13 @@ struct ufomi_chirp {
     unsigned long used;
 };
 
+// Device block kept for the batches of pipelines (ufomi_block_alloc).
+struct ufomi_block {
+    void *ptr;
+    size_t bytes;
+    int busy;
+};
+
 struct ufomi_ctx {
     int device;
     hipStream_t stream;
@@ -47,6 +54,7 @@ struct ufomi_ctx {
     hipStream_t ws_stream;
     ufomi_chirp chirps[8];   // the last used Bluestein tables (at most 96 KiB each)
     unsigned long chirp_clock;
+    ufomi_block blocks[8];   // at most 512 MiB in all, busy ones included
 };
 
 #define UFOMI_FFT_MAX 16384  // twiddle table length
@@ -65,6 +73,8 @@ int ufomi_fail(int code, const char *fmt, ...);
 
 #define UFOMI_CHECK_LAUNCH() UFOMI_HIP(hipGetLastError())
 
+// hipMalloc; when memory is short the context's idle blocks are given back first.
+hipError_t ufomi_malloc(ufomi_ctx *ctx, void **ptr, size_t bytes);
 // Device scratch owned by the context (grow-only).
 int ufomi_scratch(ufomi_ctx *ctx, size_t bytes, void **ptr);
 int ufomi_host_scratch(ufomi_ctx *ctx, size_t bytes, void **ptr);

@@ -24,6 +24,7 @@
 #include "tasks_internal.h"
 
 #include <ctype.h>
+#include <stdint.h>
 #include <stdio.h>
 #include <stdlib.h>
 #include <string.h>
@@ -180,9 +181,47 @@ static int batch_alloc(ufomi_ctx *ctx, Batch *b, const UfomiRequisition *req, in
     b->buf.req = *req;
     b->buf.dtype = dtype;
     b->buf.layout = layout;
-    int rc = ufomi_device_alloc(ctx, b->item_bytes * (size_t) (n ? n : 1), &b->buf.data);
+    int rc = ufomi_block_alloc(ctx, b->item_bytes * (size_t) (n ? n : 1), &b->buf.data);
     b->buf.owned = rc == 0;
     return rc;
+}
+
+static void batch_release(ufomi_ctx *ctx, Batch *b)
+{
+    if (b->buf.owned && b->buf.data)
+        ufomi_block_free(ctx, b->buf.data);
+    b->buf.data = NULL;
+    b->buf.owned = 0;
+}
+
+/* Where a pipeline's result goes (data NULL: the last stage's own batch) and the input it must
+ * not overlap, which every stage up to the last may read. */
+typedef struct {
+    void *data;
+    size_t capacity;
+    const void *in;
+    size_t in_bytes;
+} Dest;
+
+/* The float32 output batch of a stage that one call fills.  The last stage (to != NULL) writes
+ * the caller's memory itself where it can: the result's copy cost 0.05 ms of a 2.1 ms run (FBP of
+ * 24 slices of 1024^2) and its batch another 0.27 ms of allocation.  A result that is too large,
+ * overlaps the input, or goes to memory that is not the device's keeps its batch. */
+static int stage_alloc(ufomi_ctx *ctx, Batch *b, const UfomiRequisition *req, int n, const Dest *to)
+{
+    const size_t bytes = ufomi_requisition_elements(req) * sizeof(float) * (size_t) n;
+    if (!to || !to->data || !bytes || bytes > to->capacity || !ufomi_device_writable(ctx, to->data, bytes) ||
+        (to->in && (uintptr_t) to->in < (uintptr_t) to->data + bytes &&
+         (uintptr_t) to->data < (uintptr_t) to->in + to->in_bytes))
+        return batch_alloc(ctx, b, req, n, sizeof(float), UFOMI_F32, UFOMI_LAYOUT_REAL);
+    memset(b, 0, sizeof(*b));
+    b->n = n;
+    b->item_bytes = bytes / (size_t) n;
+    b->buf.req = *req;
+    b->buf.dtype = UFOMI_F32;
+    b->buf.layout = UFOMI_LAYOUT_REAL;
+    b->buf.data = to->data;
+    return UFOMI_OK;
 }
 
 static UfomiBuffer item_view(const Batch *b, int i)
@@ -251,7 +290,7 @@ static int read_batch(ufomi_ctx *ctx, UfomiTask *t, Batch *out, UfomiError *e)
             goto done;
         }
         if ((rc = ufomi_memcpy(ctx, out->buf.data, host, out->item_bytes * (size_t) n, 0))) {
-            ufomi_buffer_release(ctx, &out->buf);
+            batch_release(ctx, out);
             task_error(e, UFOMI_TASK_ERROR_PROCESS, rc, "read: %s", ufomi_last_error());
         }
     }
@@ -304,7 +343,7 @@ static int run_multi_input(ufomi_ctx *ctx, UfomiTask *t, const Batch *in, Batch 
     rc = ffc_task_run(t, ctx, in[0].buf.data, &in[0].buf.req, in[0].n, in[1].buf.data, in[1].n, in[2].buf.data,
                       in[2].n, out->buf.data);
     if (rc) {
-        ufomi_buffer_release(ctx, &out->buf);
+        batch_release(ctx, out);
         return task_error(e, UFOMI_TASK_ERROR_PROCESS, rc, "flat-field-correct: %s", ufomi_last_error());
     }
     t->num_processed += (unsigned) in[0].n;
@@ -314,7 +353,7 @@ static int run_multi_input(ufomi_ctx *ctx, UfomiTask *t, const Batch *in, Batch 
 /* Runs every stage but a final `write' and leaves the last batch in *res
  * (*res_owned: res holds device memory the caller releases). */
 static int run_batch(UfomiPipeline *pl, ufomi_ctx *ctx, const float *d_in, const UfomiRequisition *in_req,
-                     int n_items, Batch *res, int *res_owned, UfomiError *e)
+                     int n_items, const Dest *dest, Batch *res, int *res_owned, UfomiError *e)
 {
     const int has_read = is(pl->tasks[0], "read"), has_write = is(pl->tasks[pl->n - 1], "write");
     const int first = has_read || pl->n_branches, last = pl->n - has_write;
@@ -340,7 +379,7 @@ static int run_batch(UfomiPipeline *pl, ufomi_ctx *ctx, const float *d_in, const
         Batch br[MAX_BRANCHES];
         int owned[MAX_BRANCHES] = {0};
         for (int b = 0; b < pl->n_branches && !rc; b++)
-            rc = run_batch(pl->branches[b], ctx, NULL, NULL, 0, &br[b], &owned[b], e);
+            rc = run_batch(pl->branches[b], ctx, NULL, NULL, 0, NULL, &br[b], &owned[b], e);
         for (int b = 0; b < pl->n_branches && !rc; b++)
             if (!br[b].n)
                 rc = task_error(e, UFOMI_TASK_ERROR_PROCESS, UFOMI_ERR_ARG, "input %d of `%s' produced no items", b,
@@ -349,7 +388,7 @@ static int run_batch(UfomiPipeline *pl, ufomi_ctx *ctx, const float *d_in, const
             rc = run_multi_input(ctx, pl->tasks[0], br, &cur, e);
         for (int b = 0; b < pl->n_branches; b++)
             if (owned[b])
-                ufomi_buffer_release(ctx, &br[b].buf);
+                batch_release(ctx, &br[b]);
         if (rc)
             return rc;
         cur_owned = 1;
@@ -394,7 +433,7 @@ static int run_batch(UfomiPipeline *pl, ufomi_ctx *ctx, const float *d_in, const
             UfomiBuffer *fp[1] = {&filt};
             if ((rc = ufomi_task_get_requisition(pl->tasks[s + 2], fp, &r_ifft, e)))
                 goto out;
-            if ((rc = batch_alloc(ctx, &next, &r_ifft, cur.n, sizeof(float), UFOMI_F32, UFOMI_LAYOUT_REAL)))
+            if ((rc = stage_alloc(ctx, &next, &r_ifft, cur.n, s + 3 == last ? dest : NULL)))
                 goto fail_alloc;
             const int W = (int) cur.buf.req.dims[0];
             const int N = (int) (r_fft.dims[0] / 2);
@@ -402,7 +441,7 @@ static int run_batch(UfomiPipeline *pl, ufomi_ctx *ctx, const float *d_in, const
             rc = ufomi_ramp_filter(ctx, cur.buf.data, W, (int) rows, N, filter_task_device_coefficients(pl->tasks[s + 1]),
                                    (int) r_ifft.dims[0], next.buf.data, UFOMI_F32);
             if (rc) {
-                ufomi_buffer_release(ctx, &next.buf);
+                batch_release(ctx, &next);
                 task_error(e, UFOMI_TASK_ERROR_PROCESS, rc, "fused ramp filter: %s", ufomi_last_error());
                 goto out;
             }
@@ -413,7 +452,7 @@ static int run_batch(UfomiPipeline *pl, ufomi_ctx *ctx, const float *d_in, const
         } else if (is(t, "backproject")) {
             if ((rc = ufomi_task_get_requisition(t, ins, &req, e)))
                 goto out;
-            if ((rc = batch_alloc(ctx, &next, &req, cur.n, sizeof(float), UFOMI_F32, UFOMI_LAYOUT_REAL)))
+            if ((rc = stage_alloc(ctx, &next, &req, cur.n, s + 1 == last ? dest : NULL)))
                 goto fail_alloc;
             ufomi_bp_params bp;
             backproject_task_params(t, &bp);
@@ -421,7 +460,7 @@ static int run_batch(UfomiPipeline *pl, ufomi_ctx *ctx, const float *d_in, const
                                    (int) cur.buf.req.dims[1], cur.n, cur.item_bytes / elem_size(cur.buf.dtype), &bp,
                                    next.buf.data, 0);
             if (rc) {
-                ufomi_buffer_release(ctx, &next.buf);
+                batch_release(ctx, &next);
                 task_error(e, UFOMI_TASK_ERROR_PROCESS, rc, "backproject: %s", ufomi_last_error());
                 goto out;
             }
@@ -434,11 +473,11 @@ static int run_batch(UfomiPipeline *pl, ufomi_ctx *ctx, const float *d_in, const
                 rc = task_error(e, UFOMI_TASK_ERROR_PROCESS, UFOMI_ERR_UNSUPPORTED, "average: input must be float32");
                 goto out;
             }
-            if ((rc = batch_alloc(ctx, &next, &req, copies, sizeof(float), UFOMI_F32, UFOMI_LAYOUT_REAL)))
+            if ((rc = stage_alloc(ctx, &next, &req, copies, s + 1 == last ? dest : NULL)))
                 goto fail_alloc;
             if ((rc = ufomi_average(ctx, cur.buf.data, ufomi_requisition_elements(&req), cur.n, copies,
                                     next.buf.data))) {
-                ufomi_buffer_release(ctx, &next.buf);
+                batch_release(ctx, &next);
                 task_error(e, UFOMI_TASK_ERROR_PROCESS, rc, "average: %s", ufomi_last_error());
                 goto out;
             }
@@ -457,13 +496,13 @@ static int run_batch(UfomiPipeline *pl, ufomi_ctx *ctx, const float *d_in, const
             }
             const int W = (int) req.dims[0], number = (int) req.dims[1], H = (int) rows_of(&cur.buf.req);
             const int used = cur.n < number ? cur.n : number;
-            if ((rc = batch_alloc(ctx, &next, &req, H, sizeof(float), UFOMI_F32, UFOMI_LAYOUT_REAL)))
+            if ((rc = stage_alloc(ctx, &next, &req, H, s + 1 == last ? dest : NULL)))
                 goto fail_alloc;
             rc = ufomi_transpose_projections(ctx, cur.buf.data, W, H, used, 0, number, next.buf.data);
             if (!rc && used < number)
                 rc = ufomi_transpose_projections(ctx, NULL, W, H, number - used, used, number, next.buf.data);
             if (rc) {
-                ufomi_buffer_release(ctx, &next.buf);
+                batch_release(ctx, &next);
                 task_error(e, UFOMI_TASK_ERROR_PROCESS, rc, "transpose-projections: %s", ufomi_last_error());
                 goto out;
             }
@@ -498,7 +537,7 @@ static int run_batch(UfomiPipeline *pl, ufomi_ctx *ctx, const float *d_in, const
                 produced++;
             }
             if (t->err_status) {
-                ufomi_buffer_release(ctx, &next.buf);
+                batch_release(ctx, &next);
                 rc = task_error(e, UFOMI_TASK_ERROR_PROCESS, t->err_status, "%s", ufomi_task_last_error(t));
                 goto out;
             }
@@ -514,7 +553,7 @@ static int run_batch(UfomiPipeline *pl, ufomi_ctx *ctx, const float *d_in, const
             for (int i = 0; i < cur.n; i++) {
                 UfomiBuffer v = item_view(&cur, i), o = item_view(&next, i), *vi[1] = {&v};
                 if (!ufomi_task_process(t, vi, &o, &req)) {
-                    ufomi_buffer_release(ctx, &next.buf);
+                    batch_release(ctx, &next);
                     rc = task_error(e, UFOMI_TASK_ERROR_PROCESS, t->err_status ? t->err_status : UFOMI_ERR_ARG, "%s",
                                     ufomi_task_last_error(t));
                     goto out;
@@ -524,7 +563,7 @@ static int run_batch(UfomiPipeline *pl, ufomi_ctx *ctx, const float *d_in, const
             next.buf.layout = layout;
         }
         if (cur_owned)
-            ufomi_buffer_release(ctx, &cur.buf);
+            batch_release(ctx, &cur);
         cur = next;
         cur_owned = 1;
         continue;
@@ -538,7 +577,7 @@ static int run_batch(UfomiPipeline *pl, ufomi_ctx *ctx, const float *d_in, const
     return UFOMI_OK;
 out:
     if (cur_owned)
-        ufomi_buffer_release(ctx, &cur.buf);
+        batch_release(ctx, &cur);
     return rc;
 }
 
@@ -555,7 +594,10 @@ int ufomi_pipeline_run(UfomiPipeline *pl, ufomi_ctx *ctx, const float *d_in, con
         return task_error(e, UFOMI_TASK_ERROR_SETUP, UFOMI_ERR_ARG, "a pipeline of `read' alone has no sink");
     Batch cur;
     int cur_owned = 0;
-    int rc = run_batch(pl, ctx, d_in, in_req, n_items, &cur, &cur_owned, e);
+    Dest dest = {has_write ? NULL : d_out, out_capacity, d_in, 0};
+    if (d_in && in_req && n_items > 0)
+        dest.in_bytes = ufomi_requisition_elements(in_req) * sizeof(float) * (size_t) n_items;
+    int rc = run_batch(pl, ctx, d_in, in_req, n_items, &dest, &cur, &cur_owned, e);
     if (rc)
         return rc;
     if (has_write) {
@@ -571,7 +613,7 @@ int ufomi_pipeline_run(UfomiPipeline *pl, ufomi_ctx *ctx, const float *d_in, con
         if (total > out_capacity) {
             rc = task_error(e, UFOMI_TASK_ERROR_PROCESS, UFOMI_ERR_SIZE, "output needs %zu bytes, capacity %zu", total,
                             out_capacity);
-        } else if (total && (rc = ufomi_memcpy(ctx, d_out, cur.buf.data, total, 2))) {
+        } else if (total && cur.buf.data != d_out && (rc = ufomi_memcpy(ctx, d_out, cur.buf.data, total, 2))) {
             task_error(e, UFOMI_TASK_ERROR_PROCESS, rc, "%s", ufomi_last_error());
         } else if ((rc = ufomi_synchronize(ctx))) {
             task_error(e, UFOMI_TASK_ERROR_PROCESS, rc, "%s", ufomi_last_error());
@@ -581,6 +623,6 @@ int ufomi_pipeline_run(UfomiPipeline *pl, ufomi_ctx *ctx, const float *d_in, con
         }
     }
     if (cur_owned)
-        ufomi_buffer_release(ctx, &cur.buf);
+        batch_release(ctx, &cur);
     return rc;
 }

@@ -53,6 +53,12 @@ int task_error(UfomiError *e, int code, int status, const char *fmt, ...);
 /* Records a ufomi status + message for ufomi_last_error() and returns status. */
 int ufomi_status_fail(int status, const char *fmt, ...);
 
+/* Device blocks the context keeps between runs, for the batches of pipelines (csrc/core.hip). */
+int ufomi_block_alloc(ufomi_ctx *ctx, size_t bytes, void **out);
+int ufomi_block_free(ufomi_ctx *ctx, void *ptr);
+/* 1 when a stage's kernels may write [ptr, ptr + bytes) themselves: aligned memory of the device. */
+int ufomi_device_writable(ufomi_ctx *ctx, const void *ptr, size_t bytes);
+
 /* Helpers the pipeline uses to fuse fft ! filter ! ifft and batch backproject. */
 int fft_chain_fusable(const UfomiTask *fft, const UfomiTask *ifft, const UfomiBuffer *in);
 int filter_task_coefficients(UfomiTask *t, size_t width, UfomiError *e);

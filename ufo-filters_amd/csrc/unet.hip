@@ -18,7 +18,9 @@
 // weights, BF16 copies refreshed after every step.
 #include "ufomi_internal.h"
 #include "nn_gemm.h"
+#include "nn_wgrad.h"
 
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <string>
@@ -143,45 +145,52 @@ __global__ __launch_bounds__(256) void final_bwd_kernel(const float *__restrict_
     }
 }
 
-// Per-block column sums of a [npix][C] bf16 view (bias gradients), C <= 256
-// dividing 256: thread t sums channel t % C over pixels t / C, t / C + 256 / C, ...
+// Per-block column sums of a [npix][C] bf16 view (bias gradients), C a multiple of 8 dividing 256:
+// thread t sums the 8 channels of group t % (C / 8) over every 2048 / C-th pixel of the block.
 __global__ __launch_bounds__(256) void colsum_kernel(View<const bf16> g, long npix, int C, float *__restrict__ part)
 {
-    __shared__ float red[256];
-    const int c = threadIdx.x % C, lane = threadIdx.x / C, lanes = 256 / C;
-    float s = 0.0f;
-    for (long p = (long) blockIdx.x * lanes + lane; p < npix; p += (long) gridDim.x * lanes)
-        s += (float) *g.at(p, c);
-    red[threadIdx.x] = s;
+    __shared__ float red[256][9];
+    const int groups = C / 8, grp = threadIdx.x % groups, lane = threadIdx.x / groups, lanes = 256 / groups;
+    float s[8] = {};
+#pragma unroll 4
+    for (long p = (long) blockIdx.x * lanes + lane; p < npix; p += (long) gridDim.x * lanes) {
+        const nn::bf16x8 v = nn::ld8(g.at(p, 8 * grp));
+#pragma unroll
+        for (int e = 0; e < 8; e++) s[e] += (float) v[e];
+    }
+#pragma unroll
+    for (int e = 0; e < 8; e++) red[threadIdx.x][e] = s[e];
     __syncthreads();
     if (threadIdx.x < C) {
+        const int c8 = threadIdx.x / 8, e = threadIdx.x % 8;
         float t = 0.0f;
-        for (int k = 0; k < lanes; k++) t += red[k * C + threadIdx.x];
+        for (int k = 0; k < lanes; k++) t += red[k * groups + c8][e];
         part[(long) blockIdx.x * C + threadIdx.x] = t;
     }
 }
 
-// dst[i] = sum_z src[z * len + i] (+ dst[i] when accumulate), fixed order.
+// dst[i] = sum_z src[z * len + i] in a fixed order: a block takes 256 / Z columns, thread (z, i)
+// every Z-th partial, and the Z sums are added in LDS.  Z = 1 for few partials of many columns.
+// One pass: 256 partials of 9248 columns in 4.8 us, against 16 us as sums of 32 added again.
+template <int Z>
 __global__ __launch_bounds__(256) void reduce_kernel(const float *__restrict__ src, int nz, long len,
                                                      float *__restrict__ dst)
 {
-    const long i = (long) blockIdx.x * 256 + threadIdx.x;
-    if (i >= len) return;
+    constexpr int COLS = 256 / Z;
+    __shared__ float red[256];
+    const long i = (long) blockIdx.x * COLS + threadIdx.x % COLS;
     float s = 0.0f;
-    for (int z = 0; z < nz; z++) s += src[(long) z * len + i];
-    dst[i] = s;
-}
-
-// dst[g * len + i] = sum over z in [32 g, 32 g + 32) of src[z * len + i].
-__global__ __launch_bounds__(256) void reduce_groups_kernel(const float *__restrict__ src, int nz, long len,
-                                                            float *__restrict__ dst)
-{
-    const long i = (long) blockIdx.x * 256 + threadIdx.x;
-    if (i >= len) return;
-    const int z0 = blockIdx.y * 32, z1 = z0 + 32 < nz ? z0 + 32 : nz;
-    float s = 0.0f;
-    for (int z = z0; z < z1; z++) s += src[(long) z * len + i];
-    dst[(long) blockIdx.y * len + i] = s;
+    if (i < len) {
+#pragma unroll 4
+        for (int z = threadIdx.x / COLS; z < nz; z += Z) s += src[(long) z * len + i];
+    }
+    if constexpr (Z > 1) {
+        red[threadIdx.x] = s;
+        __syncthreads();
+        if (threadIdx.x >= COLS) return;
+        for (int z = 1; z < Z; z++) s += red[z * COLS + threadIdx.x];
+    }
+    if (i < len) dst[i] = s;
 }
 
 // 2x2 max pooling of C channels (C % 8 == 0); out grid (H/2, W/2).
@@ -599,7 +608,7 @@ int wgrad_splits(const ufomi_unet *n, long M, long N, long pixels, long *kchunk)
     const long tiles = ((M + 63) / 64) * ((N + 127) / 128);
     long splits = 2048 / tiles;
     if (splits < 1) splits = 1;
-    const long max_ws = (long) (n->ws_floats / (size_t) (M * N)) * 32 / 34;  // room for the group sums
+    const long max_ws = (long) (n->ws_floats / (size_t) (M * N));
     if (splits > max_ws) splits = max_ws;
     const long groups = (pixels + 255) / 256;  // at least 256 pixels per split
     if (splits > groups) splits = groups;
@@ -610,31 +619,71 @@ int wgrad_splits(const ufomi_unet *n, long M, long N, long pixels, long *kchunk)
     return (int) ((pixels + chunk - 1) / chunk);
 }
 
-// dst[i] = sum_z ws[z * len + i].  Many partials are first summed in groups of
-// 32 (one thread per (i, group), in parallel) into the workspace after them, so
-// no thread walks a long dependent chain; the order is fixed either way.
+// dst[i] = sum_z ws[z * len + i].
 int reduce_into(hipStream_t s, const float *ws, int nz, long len, float *dst)
 {
-    if (nz > 32) {
-        const int ng = (nz + 31) / 32;
-        float *tmp = const_cast<float *>(ws) + (long) nz * len;
-        hipLaunchKernelGGL(reduce_groups_kernel, dim3(blocks_for(len), ng), dim3(256), 0, s, ws, nz, len, tmp);
-        UFOMI_CHECK_LAUNCH();
-        ws = tmp;
-        nz = ng;
-    }
-    hipLaunchKernelGGL(reduce_kernel, dim3(blocks_for(len)), dim3(256), 0, s, ws, nz, len, dst);
+    if (nz > 256)
+        hipLaunchKernelGGL(reduce_kernel<32>, dim3((unsigned) ((len + 7) / 8)), dim3(256), 0, s, ws, nz, len, dst);
+    else if (nz > 8)
+        hipLaunchKernelGGL(reduce_kernel<8>, dim3((unsigned) ((len + 31) / 32)), dim3(256), 0, s, ws, nz, len, dst);
+    else
+        hipLaunchKernelGGL(reduce_kernel<1>, dim3(blocks_for(len)), dim3(256), 0, s, ws, nz, len, dst);
     UFOMI_CHECK_LAUNCH();
     return UFOMI_OK;
 }
 
+int bias_grad(ufomi_unet *n, hipStream_t s, View<const bf16> g, long npix, int C, float *db)
+{
+    long blocks = (npix * C + 256L * 64 - 1) / (256L * 64);
+    if (blocks < 1) blocks = 1;
+    if (blocks > 512) blocks = 512;
+    if ((size_t) (blocks * C) > n->ws_floats) blocks = (long) (n->ws_floats / C);
+    hipLaunchKernelGGL(colsum_kernel, dim3((unsigned) blocks), dim3(256), 0, s, g, npix, C, n->ws);
+    UFOMI_CHECK_LAUNCH();
+    return reduce_into(s, n->ws, (int) blocks, C, db);
+}
+
+// Units of rows and workgroups per channel tile of the NHWC weight gradients: the shortest units
+// (at least 2 rows; R rows stage R + 2) that give each of the 256 CUs at most one workgroup, and
+// no more partials of `len` floats than the workspace holds.
+void wgrad_units(const ufomi_unet *n, int B, int lh, int lw, long tiles, long len, int *lr, int *units, int *splits)
+{
+    long u, sp;
+    for (*lr = 1;; ++*lr) {
+        u = ((long) B << (lw - 5)) << (lh - *lr);
+        sp = (u + nn::kWgWaves - 1) / nn::kWgWaves;
+        if (*lr >= lh || tiles * sp <= 256) break;
+    }
+    sp = std::min(sp, std::max(1L, 256 / tiles));
+    *units = (int) u;
+    *splits = (int) std::min(sp, (long) (n->ws_floats / (size_t) len));
+}
+
+// Weight and bias gradients (dw, and db = dw + 9 cin cout behind it) of one conv.
 int conv3_wgrad(ufomi_unet *n, hipStream_t s, View<const bf16> g, View<const bf16> in, long npix, int l, int cin,
                 int cout, float *dw)
 {
     const long M = cout, N = 9L * cin;
+    const int lh = n->lh - l, lw = n->lw - l;
+    if (lw >= 5) {  // strips of 32 pixels; narrower levels take the channel-major product
+        const int B = (int) (npix >> (lh + lw));
+        const long len = M * N + cout, tiles = cin == 1 ? 1 : (cout / 32) * (long) (cin / 32);
+        int lr, units, splits;
+        wgrad_units(n, B, lh, lw, tiles, len, &lr, &units, &splits);
+        const dim3 grid((unsigned) (tiles * splits)), block(nn::kWgWaves * 64);
+        if (cin == 1)
+            hipLaunchKernelGGL(nn::wgrad_first_kernel, grid, block, 0, s,
+                               nn::WgradFirst{g, in.ptr, lh, lw, lr, units, splits, n->ws});
+        else
+            hipLaunchKernelGGL(nn::wgrad3_kernel, grid, block, 0, s,
+                               nn::Wgrad3{g, in, lh, lw, lr, cin, cout, units, splits, n->ws});
+        UFOMI_CHECK_LAUNCH();
+        return reduce_into(s, n->ws, splits, len, dw);
+    }
+    int rc = bias_grad(n, s, g, npix, cout, dw + M * N);
+    if (rc) return rc;
     long chunk;
     const int splits = wgrad_splits(n, M, N, npix, &chunk);
-    const int lh = n->lh - l, lw = n->lw - l;
     const size_t need = (size_t) (cout + 3 * cin) * (size_t) npix;
     if (lw >= 3 && n->wgT && need <= n->wgT_elems && npix % kTpPix == 0) {
         // channel-major copies (g, and the input at the three row shifts), then 16-byte fragments
@@ -653,8 +702,7 @@ int conv3_wgrad(ufomi_unet *n, hipStream_t s, View<const bf16> g, View<const bf1
         op.cout = cout;
         op.npix = npix;
         op.part = nn::Partial{n->ws, M, N, chunk, npix};
-        int rc = gemm_wgrad(s, op, M, N, splits);
-        if (rc) return rc;
+        if ((rc = gemm_wgrad(s, op, M, N, splits))) return rc;
         return reduce_into(s, n->ws, splits, M * N, dw);
     }
     nn::Conv3Wgrad op;
@@ -666,20 +714,8 @@ int conv3_wgrad(ufomi_unet *n, hipStream_t s, View<const bf16> g, View<const bf1
     op.cout = cout;
     op.npix = npix;
     op.part = nn::Partial{n->ws, M, N, chunk, npix};
-    int rc = gemm_wgrad(s, op, M, N, splits);
-    if (rc) return rc;
+    if ((rc = gemm_wgrad(s, op, M, N, splits))) return rc;
     return reduce_into(s, n->ws, splits, M * N, dw);
-}
-
-int bias_grad(ufomi_unet *n, hipStream_t s, View<const bf16> g, long npix, int C, float *db)
-{
-    long blocks = (npix * C + 256L * 64 - 1) / (256L * 64);
-    if (blocks < 1) blocks = 1;
-    if (blocks > 4096) blocks = 4096;
-    if ((size_t) (blocks * C) > n->ws_floats) blocks = (long) (n->ws_floats / C);
-    hipLaunchKernelGGL(colsum_kernel, dim3((unsigned) blocks), dim3(256), 0, s, g, npix, C, n->ws);
-    UFOMI_CHECK_LAUNCH();
-    return reduce_into(s, n->ws, (int) blocks, C, db);
 }
 
 int maxpool(hipStream_t s, View<const bf16> in, View<bf16> out, long nout, int lh, int lw, int C)
@@ -812,13 +848,11 @@ int backward(ufomi_unet *n, hipStream_t s, const float *img, const float *tgt, i
         const ConvP &a = n->dec1[l], &b = n->dec2[l], &u = n->up[l];
         // d2 = relu(conv(d1))
         if ((rc = conv3_wgrad(n, s, cv(n->g_d2[l], C), cv(n->d1[l], C), np, l, C, C, g + b.w)) ||
-            (rc = bias_grad(n, s, cv(n->g_d2[l], C), np, C, g + b.b)) ||
             (rc = conv3(n, s, cv(n->g_d2[l], C), np, l, C, C, n->wtrans + b.wt, nullptr, false, cv(n->d1[l], C), 0,
                         mv(n->g_d1[l], C))))
             return rc;
         // d1 = relu(conv(cat)), cat = [up | skip]: plain data gradient of the concatenation
         if ((rc = conv3_wgrad(n, s, cv(n->g_d1[l], C), cv(n->cat[l], 2 * C), np, l, 2 * C, C, g + a.w)) ||
-            (rc = bias_grad(n, s, cv(n->g_d1[l], C), np, C, g + a.b)) ||
             (rc = conv3(n, s, cv(n->g_d1[l], C), np, l, C, 2 * C, n->wtrans + a.wt, nullptr, false, cv(nullptr, 0),
                         0, mv(n->g_cat[l], 2 * C))))
             return rc;
@@ -869,7 +903,6 @@ int backward(ufomi_unet *n, hipStream_t s, const float *img, const float *tgt, i
         const ConvP &c2 = n->enc2[l], &c1 = n->enc1[l];
         // skip_l (or bottom) = relu(conv(e1))
         if ((rc = conv3_wgrad(n, s, cv(n->g_e2[l], C), cv(n->e1[l], C), np, l, C, C, g + c2.w)) ||
-            (rc = bias_grad(n, s, cv(n->g_e2[l], C), np, C, g + c2.b)) ||
             (rc = conv3(n, s, cv(n->g_e2[l], C), np, l, C, C, n->wtrans + c2.wt, nullptr, false, cv(n->e1[l], C), 0,
                         mv(n->g_e1[l], C))))
             return rc;
@@ -877,15 +910,12 @@ int backward(ufomi_unet *n, hipStream_t s, const float *img, const float *tgt, i
             // e1 = relu(conv(pool_{l-1})); pool values are maxima of ReLU outputs, the
             // gradient goes on to the pooling (no mask here)
             if ((rc = conv3_wgrad(n, s, cv(n->g_e1[l], C), cv(n->pool[l - 1], C / 2), np, l, C / 2, C, g + c1.w)) ||
-                (rc = bias_grad(n, s, cv(n->g_e1[l], C), np, C, g + c1.b)) ||
                 (rc = conv3(n, s, cv(n->g_e1[l], C), np, l, C, C / 2, n->wtrans + c1.wt, nullptr, false,
                             cv(nullptr, 0), 0, mv(n->g_pool[l - 1], C / 2))))
                 return rc;
         } else {
             const ConvP &f = n->first;
-            if ((rc = conv3_wgrad(n, s, cv(n->g_e1[0], C), cv(n->img16, 1), np, 0, 1, C, g + f.w)) ||
-                (rc = bias_grad(n, s, cv(n->g_e1[0], C), np, C, g + f.b)))
-                return rc;
+            if ((rc = conv3_wgrad(n, s, cv(n->g_e1[0], C), cv(n->img16, 1), np, 0, 1, C, g + f.w))) return rc;
         }
     }
     return UFOMI_OK;
@@ -1030,10 +1060,11 @@ extern "C" int ufomi_unet_create(ufomi_ctx *ctx, int max_batch, int height, int 
         }
         n->ws_floats = 32u << 20;  // 128 MiB of split-K partial sums
         if (!rc) rc = dalloc_t(n, n->ws_floats, &n->ws);
-        // channel-major operand copies of the largest weight gradient: (cout + 3 cin) x pixels
+        // channel-major operand copies of the largest narrow level's weight gradient: (cout + 3 cin) x pixels
         size_t wg = 0;
         auto need = [&](const ConvP &c, int l) {
-            wg = std::max(wg, (size_t) (c.cout + 3 * c.cin) * (size_t) npix_at(n, max_batch, l));
+            if (n->lw - l < 5)  // the other levels read NHWC
+                wg = std::max(wg, (size_t) (c.cout + 3 * c.cin) * (size_t) npix_at(n, max_batch, l));
         };
         need(n->first, 0);
         for (int l = 0; l < kLevels; l++) {

@@ -554,44 +554,51 @@ int conv3(ufomi_unet *n, hipStream_t s, View<const bf16> in, long npix, int l, i
     op.out = out;
     op.pool = pool;
     const int lh = n->lh - l, lw = n->lw - l;
+    // the staging loads and the 16-byte stores of the smaller tiles need aligned tensors
+    const bool aligned = ((uintptr_t) in.ptr | (uintptr_t) w | (uintptr_t) out.ptr) % 16 == 0;
+    if ((lw >= 6 || (lw == 5 && aligned)) && lh >= 3) {
+        // LDS-staged patches of 8 rows x 64 or 32 pixels, 64 or 32 output channels per workgroup,
+        // in one flat grid of pixel tiles x channel tiles.  Larger tiles read the patch and the
+        // weights less often, but a workgroup waits for each 32-channel chunk it stages: below
+        // two workgroups per CU, which hide each other's waits, the next smaller tile is faster
+        // (forward of 8 images of 256^2 with the lines at 1, 256, 512 and 1024 workgroups: 415,
+        // 371, 334 and 332 us; of 16 images of 512^2: 1874, 1873, 1869 and 1900 us).
+        constexpr long kConvGrid = 512;
+        auto grid = [&](int nt, int tx) { return (npix / (8 * tx)) * ((cout + 16 * nt - 1) / (16 * nt)); };
+        auto launch = [&](auto kern, int nt, int tx) {
+            if (grid(nt, tx) > 0x7fffffffL) return ufomi_fail(UFOMI_ERR_SIZE, "conv grid too large");
+            hipLaunchKernelGGL(kern, dim3((unsigned) grid(nt, tx)), dim3(256), 0, s, op);
+            UFOMI_CHECK_LAUNCH();
+            return (int) UFOMI_OK;
+        };
+        if (fin && cout == 32) {
+            op.fin_w = fin->w;
+            op.fin_b = fin->b;
+            op.fin_img = fin->img;
+            op.fin_out = fin->out;
+            if (!fin->keep_d) op.out.ptr = nullptr;
+            *fused = true;
+        }
+        if (cout <= 32 || (aligned && grid(4, 32) < kConvGrid)) return launch(nn::conv3_t8_kernel<2, true, 2, 32>, 2, 32);
+        if (lw == 5 || (aligned && grid(4, 64) < kConvGrid))
+            return pool.ptr ? launch(nn::conv3_t8_kernel<4, true, 2, 32>, 4, 32)
+                            : launch(nn::conv3_t8_kernel<4, false, 2, 32>, 4, 32);
+        return pool.ptr ? launch(nn::conv3_t8_kernel<4, true, 2>, 4, 64)
+                        : launch(nn::conv3_t8_kernel<4, false, 2>, 4, 64);
+    }
     if (lw >= 6 && lh >= 2) {
-        // LDS-staged input patches (8 or 4 rows x 64 pixels per workgroup)
+        // images of 4 rows: patches of 4 rows x 64 pixels
         const long tiles = npix >> 8;
         const int NT = cout <= 32 ? 2 : 4;
         const long gy = (cout + 16 * NT - 1) / (16 * NT);
         if (tiles > 0x7fffffffL || gy > 65535)
             return ufomi_fail(UFOMI_ERR_SIZE, "conv grid too large");
-        // 32 output channels and pooled outputs leave through LDS in 16-byte vectors; for 64
-        // channels per workgroup the direct 8-byte stores measured faster.  Images of at least
-        // 8 rows take the 8-row tiles, 32 pixels wide for 32 output channels (measured: forward
-        // 34.2 ms against 34.7 ms with 64-pixel tiles and L2 weight fragments).
-        auto launch = [&](auto kern, long nt) {
-            hipLaunchKernelGGL(kern, dim3((unsigned) nt, (unsigned) gy), dim3(256), 0, s, op);
+        auto launch = [&](auto kern) {
+            hipLaunchKernelGGL(kern, dim3((unsigned) tiles, (unsigned) gy), dim3(256), 0, s, op);
         };
-        // the 8-row kernel takes one flat grid of pixel tiles x channel tiles (at most `tiles` of
-        // them, the 4-row count)
-        if (lh >= 3 && tiles * gy > 0x7fffffffL)
-            return ufomi_fail(UFOMI_ERR_SIZE, "conv grid too large");
-        auto launch8 = [&](auto kern, long nt) {
-            hipLaunchKernelGGL(kern, dim3((unsigned) (nt * gy)), dim3(256), 0, s, op);
-        };
-        if (lh >= 3) {
-            if (fin && cout == 32) {
-                op.fin_w = fin->w;
-                op.fin_b = fin->b;
-                op.fin_img = fin->img;
-                op.fin_out = fin->out;
-                if (!fin->keep_d) op.out.ptr = nullptr;
-                *fused = true;
-            }
-            if (NT == 2) launch8(nn::conv3_t8_kernel<2, true, 2, 32>, tiles);
-            else if (pool.ptr) launch8(nn::conv3_t8_kernel<4, true, 2>, tiles / 2);
-            else launch8(nn::conv3_t8_kernel<4, false, 2>, tiles / 2);
-        } else {
-            if (NT == 2) launch(nn::conv3_lds_kernel<2, true>, tiles);
-            else if (pool.ptr) launch(nn::conv3_lds_kernel<4, true>, tiles);
-            else launch(nn::conv3_lds_kernel<4, false>, tiles);
-        }
+        if (NT == 2) launch(nn::conv3_lds_kernel<2, true>);
+        else if (pool.ptr) launch(nn::conv3_lds_kernel<4, true>);
+        else launch(nn::conv3_lds_kernel<4, false>);
         UFOMI_CHECK_LAUNCH();
         return UFOMI_OK;
     }

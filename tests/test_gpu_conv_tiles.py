@@ -51,3 +51,26 @@ def test_batches_take_other_tiles_and_agree(ctx, torch_dev):
             net.forward(img[i:i + 1].contiguous(), one[i:i + 1])
         assert torch.equal(out[:n], one[:n]), n
     net.close()
+
+
+# transposed convolutions whose pixels do not fill the tiles of 128 (20, 80 and 320 of them), cross
+# images within a tile, and (8 x 64 x 64: 4096) take the XCD order
+@pytest.mark.parametrize("B,H,W", [(5, 16, 16), (3, 16, 64), (8, 64, 64)])
+def test_transposed_conv_tiles(ctx, torch_dev, B, H, W):
+    import torch
+    params = U.random_params(np.random.default_rng(29))
+    net = ufomi.Unet(ctx, B, H, W)
+    flat = np.zeros(net.padded, dtype=np.float32)
+    for name, off, dims in net.tensors:
+        flat[off:off + int(np.prod(dims))] = params[name].reshape(-1)
+    net.set_params(flat)
+    img = np.random.default_rng(30).standard_normal((B, H, W)).astype(np.float32)
+    d_in = torch.from_numpy(img).to(torch_dev)
+    out = torch.full((B + 1, H, W), 7.0, device=torch_dev)
+    net.forward(d_in, out[:B])
+    assert bool((out[B] == 7.0).all())
+    ref, _ = U.UNet(params).forward(img.astype(np.float64))
+    r32, _ = U.UNet(params, acc=np.float32).forward(img.astype(np.float64))
+    # three times what float32 accumulation does through the bf16 layers
+    assert rel_l2(out[:B].cpu().numpy() - img, ref - img) < 3 * rel_l2(r32 - img, ref - img) + 2e-3
+    net.close()

@@ -37,6 +37,13 @@ __device__ __forceinline__ bf16x8 zero8()
 
 __device__ __forceinline__ bf16x8 ld8(const bf16 *p) { return *reinterpret_cast<const bf16x8 *>(p); }
 
+// 16 bytes from each lane's address to LDS address dst (uniform) + 16 lane, in flight until the
+// caller's vmcnt wait; the builtin would wait before the next LDS read.
+__device__ __forceinline__ void load_lds_async(unsigned dst, const void *src)
+{
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(dst), "v"(src) : "memory");
+}
+
 // Workgroup of 256 threads = WM x WN waves; each wave owns MT x NT tiles of
 // 16 x 16.  Fragments of step k+32 are loaded before the MFMAs of step k.
 template <int MT, int NT, int WM, int WN, typename Op>
@@ -82,13 +89,8 @@ __global__ __launch_bounds__(256) void gemm_kernel(Op op)
 #pragma unroll
             for (int i = 0; i < MT; i++)
 #pragma unroll
-                for (int j = 0; j < NT; j++) {
-                    // kVecStore: B as the row operand, so a lane receives 4 consecutive columns of one row
-                    if constexpr (Op::kVecStore)
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[j], a[i], acc[i][j], 0, 0, 0);
-                    else
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
-                }
+                for (int j = 0; j < NT; j++)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
             if (more) {
 #pragma unroll
                 for (int i = 0; i < MT; i++) a[i] = an[i];
@@ -97,48 +99,13 @@ __global__ __launch_bounds__(256) void gemm_kernel(Op op)
             }
         }
     }
-    if constexpr (Op::kVecStore) {
-        // finished bf16 values through LDS (D[4q + e][r] of tile (i, j) is column n0 + 16 j + 4 q + e
-        // of row m0 + 16 i + r: one 8-byte write per tile), then 16-byte stores of 8 consecutive
-        // columns; a tile wholly inside M x N skips the per-element bounds tests, and the stores
-        // address from a per-tile base with 32-bit offsets
-        __shared__ bf16x8 tile[BM * BN / 8];
-        bf16 *t = reinterpret_cast<bf16 *>(tile);
-        const int mw = (wave % WM) * MT * 16, nw = (wave / WM) * NT * 16;
-        const long mb = (long) blockIdx.x * BM, nb = (long) blockIdx.y * BN;
-        const bool full = op.inside(mb + BM - 1, nb + BN - 1);
 #pragma unroll
-        for (int j = 0; j < NT; j++) {
-            // the 4 columns' bias, loaded once and unconditionally (loads under the bounds
-            // test would each wait on their own)
-            const long n = n0 + j * 16 + 4 * q;
-            const f32x4 bj = op.bias4(n);
+    for (int i = 0; i < MT; i++)
 #pragma unroll
-            for (int i = 0; i < MT; i++) {
-                const long m = m0 + i * 16 + r;
-                bf16x4 o;
+        for (int j = 0; j < NT; j++)
 #pragma unroll
-                for (int e = 0; e < 4; e++)
-                    o[e] = (bf16) (full || op.valid(m, n + e) ? acc[i][j][e] + bj[e] : 0.0f);
-                *reinterpret_cast<bf16x4 *>(t + (mw + i * 16 + r) * BN + nw + j * 16 + 4 * q) = o;
-            }
-        }
-        __syncthreads();
-        const typename Op::TileBase tb = op.tile_base(mb);
-        for (int v = threadIdx.x; v < BM * BN / 8; v += 256) {
-            const int lm = v / (BN / 8);
-            const long n = nb + (v % (BN / 8)) * 8;
-            if (full || op.valid(mb + lm, n)) op.store8(tb, lm, (int) n, tile[v]);
-        }
-    } else {
-#pragma unroll
-        for (int i = 0; i < MT; i++)
-#pragma unroll
-            for (int j = 0; j < NT; j++)
-#pragma unroll
-                for (int e = 0; e < 4; e++)
-                    op.store(m0 + i * 16 + 4 * q + e, n0 + j * 16 + r, acc[i][j][e], blockIdx.z);
-    }
+            for (int e = 0; e < 4; e++)
+                op.store(m0 + i * 16 + 4 * q + e, n0 + j * 16 + r, acc[i][j][e], blockIdx.z);
 }
 
 // A tensor of pixels in NHWC order: element (pixel p, channel c) at
@@ -167,7 +134,6 @@ __device__ __forceinline__ Pix pix_of(long p, int lh, int lw)
 // zero padding, K ordered (tap, c); cin a multiple of 32.  With mask, channels
 // n >= mask_from are zeroed where mask[p][n] <= 0 (a ReLU derivative).
 struct Conv3 {
-    static constexpr bool kVecStore = false;
     View<const bf16> in;
     int lh, lw, lcin, cout;
     long npix;
@@ -281,91 +247,132 @@ struct Conv3 {
 // pixels, N = 4 cout ((ab, co)), K = cin (multiple of 32).  Output grid is
 // (2h, 2w).
 struct UpFwd {
-    // outputs leave as 8 consecutive channels (cout a multiple of 8) of one child pixel
-    static constexpr bool kVecStore = true;
     View<const bf16> in;
-    int lh, lw, lcin, lcout;
+    int lh, lw, cin, lcout;  // cin a multiple of 64, 4 cout of 128
     long npix;
     const bf16 *w;      // [4][cout][cin]
     const float *bias;  // [cout]
     View<bf16> out;
-
-    struct RowA {
-        long p;
-        bool ok;
-    };
-    struct ColB {
-        const bf16 *w;
-        bool ok;
-    };
-    __device__ __forceinline__ RowA row_a(long m) const { return RowA{m, m < npix}; }
-    __device__ __forceinline__ ColB col_b(long n) const
-    {
-        const bool ok = n < (4L << lcout);
-        return ColB{w + ((ok ? n : 0) << lcin), ok};
-    }
-    __device__ __forceinline__ void k_range(int, long &k0, long &k1) const
-    {
-        k0 = 0;
-        k1 = 1L << lcin;
-    }
-    __device__ __forceinline__ bf16x8 load_a(const RowA &r, long k) const
-    {
-        return r.ok ? ld8(in.at(r.p, (int) k)) : zero8();
-    }
-    __device__ __forceinline__ bf16x8 load_b(const ColB &c, long k) const { return c.ok ? ld8(c.w + k) : zero8(); }
-    __device__ __forceinline__ bool valid(long m, long n) const { return m < npix && n < (4L << lcout); }
-    __device__ __forceinline__ bool inside(long m, long n) const { return valid(m, n); }
-    __device__ __forceinline__ float finish(long, long n, float v) const
-    {
-        return v + bias[n & ((1 << lcout) - 1)];
-    }
-    // bias of columns n .. n + 3 (n a multiple of 4; any n, as finish reads it)
-    __device__ __forceinline__ f32x4 bias4(long n) const
-    {
-        const float *b = bias + (n & ((1 << lcout) - 1));
-        return f32x4{b[0], b[1], b[2], b[3]};
-    }
-    // Output base of the image holding input pixel mb, and mb's (y, x): the children of input
-    // pixel mb + lm are then 32-bit offsets from it (a tile's rows run on into the next image
-    // contiguously; 8 h w cs < 2^32, checked on the host).
-    struct TileBase {
-        bf16 *img0;
-        int y0, x0;
-    };
-    __device__ __forceinline__ TileBase tile_base(long mb) const
-    {
-        const long img = mb >> (lh + lw);
-        const Pix px = pix_of(mb, lh, lw);
-        return TileBase{out.ptr + (img << (lh + lw + 2)) * out.cs + out.c0, px.y, px.x};
-    }
-    __device__ __forceinline__ long child(long m, int ab) const
-    {
-        const long img = m >> (lh + lw);
-        const Pix px = pix_of(m, lh, lw);
-        return (((img << (lh + 1)) + 2 * px.y + (ab >> 1)) << (lw + 1)) + 2 * px.x + (ab & 1);
-    }
-    // columns n .. n + 7 of input pixel tb + lm (one child pixel)
-    __device__ __forceinline__ void store8(const TileBase &tb, int lm, int n, bf16x8 v) const
-    {
-        const int ab = n >> lcout, co = n & ((1 << lcout) - 1);
-        const int xx = tb.x0 + lm, x = xx & ((1 << lw) - 1), y = tb.y0 + (xx >> lw);
-        const unsigned c = (unsigned) ((((2 * y + (ab >> 1)) << (lw + 1)) + 2 * x + (ab & 1)));
-        *reinterpret_cast<bf16x8 *>(tb.img0 + c * (unsigned) out.cs + (unsigned) co) = v;
-    }
-    __device__ __forceinline__ void store(long m, long n, float v, int) const
-    {
-        if (!valid(m, n)) return;
-        const int ab = (int) (n >> lcout), co = (int) (n & ((1 << lcout) - 1));
-        *out.at(child(m, ab), co) = (bf16) finish(m, n, v);
-    }
 };
+
+// A workgroup of 4 waves computes 128 input pixels x 128 of the 4 cout columns, a wave 64 x 64.
+// Chunks of 64 input channels of both operands go to LDS in 16-byte pieces (piece c of row m at
+// position c ^ m % 8, so the 16 rows of a fragment lie in different banks), with NB = 2 a chunk
+// ahead; cin = 64 is one chunk, and half the LDS lets twice the workgroups in.  Weights are the
+// row operand, so a lane gets 4 consecutive columns; the finished tile leaves through LDS in
+// 16-byte stores of 8 channels of a child pixel.
+//
+// Bound by memory at 64 channels (in 128 B and out 256 B a pixel) and by the waits for the chunks
+// above.  16 images of 512^2: 46, 68 and 111 us for 256, 128 and 64 channels, against 79, 106 and
+// 155 us with fragments loaded from memory straight into registers.
+template <int NB>
+__global__ __launch_bounds__(256) void up_fwd_kernel(UpFwd op)
+{
+    constexpr int BM = 128, BN = 128, CHUNK = (BM + BN) * 128;  // bytes
+    __shared__ __align__(16) char lds[NB * CHUNK];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r = lane & 15, q = lane >> 4;
+    const int mw = (wave & 1) * 64, nw = (wave >> 1) * 64;
+    // flat grid; the column tiles of a pixel tile follow each other on one XCD and find its pixels
+    // in that L2 (where the pixel tiles divide by 8)
+    const int gy = (4 << op.lcout) / BN, gx = gridDim.x / gy;
+    int bx, by;
+    if ((gx & 7) == 0) {
+        const int slot = (int) blockIdx.x >> 3;
+        bx = ((int) blockIdx.x & 7) * (gx / 8) + slot / gy;
+        by = slot % gy;
+    } else {
+        bx = (int) blockIdx.x / gy;
+        by = (int) blockIdx.x % gy;
+    }
+    const long mb = (long) bx * BM;
+    const int nb = by * BN;
+
+    // this wave's pieces of a chunk: 8 rows of 8 pieces a load, 4 loads of each operand
+    const bf16 *src[8];
+    const int piece = 8 * ((lane & 7) ^ (lane >> 3));
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        const int row = (wave * 4 + k) * 8 + (lane >> 3);
+        src[k] = op.in.at(mb + row < op.npix ? mb + row : op.npix - 1, piece);  // past the end: not stored
+        src[4 + k] = op.w + (long) (nb + row) * op.cin + piece;
+    }
+    const unsigned base = (unsigned) (uintptr_t) (__attribute__((address_space(3))) char *) lds;
+    auto stage = [&](int c) {
+        const unsigned dst = base + (NB > 1 ? c & 1 : 0) * CHUNK + wave * 4096;
+#pragma unroll
+        for (int k = 0; k < 8; k++) load_lds_async(dst + (k >> 2) * (BM * 128) + (k & 3) * 1024, src[k] + 64 * c);
+    };
+    f32x4 acc[4][4];
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    const int chunks = op.cin / 64;
+    stage(0);
+    for (int c = 0; c < chunks; c++) {
+        if (NB > 1 && c + 1 < chunks) {
+            stage(c + 1);
+            asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+        } else {
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        }
+        __syncthreads();  // every wave's part of chunk c is in LDS
+        const char *a0 = lds + (NB > 1 ? c & 1 : 0) * CHUNK, *b0 = a0 + BM * 128;
+#pragma unroll
+        for (int k = 0; k < 2; k++) {
+            const int pos = 16 * ((4 * k + q) ^ (r & 7));
+            bf16x8 a[4], b[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                a[i] = *reinterpret_cast<const bf16x8 *>(a0 + (mw + 16 * i + r) * 128 + pos);
+                b[i] = *reinterpret_cast<const bf16x8 *>(b0 + (nw + 16 * i + r) * 128 + pos);
+            }
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[j], a[i], acc[i][j], 0, 0, 0);
+        }
+        __syncthreads();  // chunk c has been read; its buffer is staged again, or takes the tile below
+        if (NB == 1 && c + 1 < chunks) stage(c + 1);
+    }
+    // D[4 q + e][r] of tile (i, j): column nw + 16 j + 4 q + e of pixel mw + 16 i + r
+    bf16 *t = reinterpret_cast<bf16 *>(lds);
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const int n = nw + 16 * j + 4 * q;
+        const float *b = op.bias + ((nb + n) & ((1 << op.lcout) - 1));
+        const f32x4 bj = {b[0], b[1], b[2], b[3]};
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const f32x4 v = acc[i][j] + bj;
+            bf16x4 o;
+#pragma unroll
+            for (int e = 0; e < 4; e++) o[e] = (bf16) v[e];
+            *reinterpret_cast<bf16x4 *>(t + (mw + 16 * i + r) * BN + n) = o;
+        }
+    }
+    __syncthreads();
+    // Children of input pixel mb + lm as 32-bit offsets from the image holding mb (a tile's rows run
+    // on into the next image contiguously; 8 h w cs < 2^32, checked on the host).
+    const Pix p0 = pix_of(mb, op.lh, op.lw);
+    bf16 *img0 = op.out.ptr + ((mb >> (op.lh + op.lw)) << (op.lh + op.lw + 2)) * op.out.cs + op.out.c0;
+    for (int v = threadIdx.x; v < BM * BN / 8; v += 256) {
+        const int lm = v / (BN / 8), n = nb + (v % (BN / 8)) * 8;
+        if (mb + lm >= op.npix) break;  // lm grows with v
+        const int ab = n >> op.lcout, co = n & ((1 << op.lcout) - 1);
+        const int xx = p0.x + lm, x = xx & ((1 << op.lw) - 1), y = p0.y + (xx >> op.lw);
+        const unsigned child = (unsigned) (((2 * y + (ab >> 1)) << (op.lw + 1)) + 2 * x + (ab & 1));
+        *reinterpret_cast<bf16x8 *>(img0 + child * (unsigned) op.out.cs + (unsigned) co) =
+            *reinterpret_cast<const bf16x8 *>(t + v * 8);
+    }
+}
 
 // Data gradient of UpFwd: gin[p][c] = sum_{ab, co} g[child(p, ab)][co] wT[c][ab][co],
 // masked by the ReLU of the forward input.  M = input pixels, N = cin,
 // K = 4 cout ((ab, co), cout a multiple of 32).
 struct UpDgrad {
-    static constexpr bool kVecStore = false;
     View<const bf16> g;
     int lh, lw, lcout, cin;
     long npix;
@@ -440,7 +447,6 @@ struct Partial {
 // M = cout, N = 9 cin ((tap, c)), K = pixels in groups of 8 along a row
 // (W a multiple of 8).  Pixel-strided operands: 8 scalar loads per fragment.
 struct Conv3Wgrad {
-    static constexpr bool kVecStore = false;
     View<const bf16> g;
     View<const bf16> in;
     int lh, lw, cin, cout;
@@ -502,7 +508,6 @@ struct Conv3Wgrad {
 // The tap's row shift dy is an offset of dy W pixels, zero where y + dy leaves
 // the image.
 struct Conv3WgradT {
-    static constexpr bool kVecStore = false;
     const bf16 *gT;
     const bf16 *inT;
     int lh, lw, cin, cout;
@@ -551,7 +556,6 @@ struct Conv3WgradT {
 // Weight gradient of UpFwd: dW[ab][co][c] = sum_p g[child(p, ab)][co] in[p][c].
 // M = 4 cout ((ab, co)), N = cin, K = input pixels (groups of 8 along a row).
 struct UpWgrad {
-    static constexpr bool kVecStore = false;
     View<const bf16> g;
     View<const bf16> in;
     int lh, lw, lcout, cin;

@@ -40,13 +40,6 @@ struct Wgrad3 {
     float *part;    // [splits][cout][9][cin], then cout bias sums, per split
 };
 
-// 16 bytes from each lane's address to LDS address dst (uniform) + 16 lane, in flight until the
-// caller's vmcnt wait; the builtin would wait before the next LDS read.
-__device__ __forceinline__ void wg_load_lds(unsigned dst, const void *src)
-{
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(dst), "v"(src) : "memory");
-}
-
 typedef __attribute__((address_space(3))) char wg_lds_char;
 
 // The fragment of 32 pixels x 16 channels at LDS address a: pixels 4 q .. 4 q + 3 and 16 + the same.
@@ -96,12 +89,12 @@ __global__ __launch_bounds__(kWgWaves * 64) void wgrad3_kernel(Wgrad3 op)
             const bool gok = i < R, xok = i < R + 2 && ya - 1 + i >= 0 && ya - 1 + i < H;
             const bf16 *gs = gp + i * g_row, *xs = xp + i * x_row;
             const void *z = &wg_zeros;
-            wg_load_lds(dst, gok ? gs : z);
-            wg_load_lds(dst + 1024, gok ? gs + 16 * op.g.cs : z);
-            wg_load_lds(dst + kWgG, xok && left ? xs : z);
-            wg_load_lds(dst + kWgG + 1024, xok ? xs + 16 * op.in.cs : z);
+            load_lds_async(dst, gok ? gs : z);
+            load_lds_async(dst + 1024, gok ? gs + 16 * op.g.cs : z);
+            load_lds_async(dst + kWgG, xok && left ? xs : z);
+            load_lds_async(dst + kWgG + 1024, xok ? xs + 16 * op.in.cs : z);
             // pixels 32 and 33 (one lane in four of 8: the same channels as pixels 0 and 1)
-            if (lane < 8) wg_load_lds(dst + kWgG + 2048, xok && right ? xs + 32 * op.in.cs : z);
+            if (lane < 8) load_lds_async(dst + kWgG + 2048, xok && right ? xs + 32 * op.in.cs : z);
         };
         // Fragment addresses within a slot: this lane's pixel 4 q + l16 / 4, 4 channels.
         auto address = [&](int p) { return p * 64 + 16 * ((l16 & 3) >> 1) + 8 * (l16 & 1) + 32 * (p >> 2 & 1); };

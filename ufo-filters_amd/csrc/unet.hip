@@ -786,7 +786,7 @@ int forward(ufomi_unet *n, hipStream_t s, const float *img, int B, float *out)
         up.in = cv(src, 2 * C);
         up.lh = n->lh - l - 1;
         up.lw = n->lw - l - 1;
-        up.lcin = ilog2(2 * C);
+        up.cin = 2 * C;
         up.lcout = ilog2(C);
         up.npix = npix_at(n, B, l + 1);
         up.w = n->w16 + n->up[l].w;
@@ -795,7 +795,11 @@ int forward(ufomi_unet *n, hipStream_t s, const float *img, int B, float *out)
         if ((8L << (up.lh + up.lw)) * up.out.cs >= (1L << 32))
             return ufomi_fail(UFOMI_ERR_SIZE, "transposed conv output of %ld pixels x %d channels exceeds 32-bit offsets",
                               4L << (up.lh + up.lw), up.out.cs);
-        if ((rc = gemm_fwd(s, up, up.npix, 4L * C))) return rc;
+        const long tiles = ((up.npix + 127) / 128) * (4 * C / 128);
+        if (tiles > 0x7fffffffL) return ufomi_fail(UFOMI_ERR_SIZE, "transposed conv grid too large");
+        hipLaunchKernelGGL(up.cin == 64 ? nn::up_fwd_kernel<1> : nn::up_fwd_kernel<2>, dim3((unsigned) tiles), dim3(256),
+                           0, s, up);
+        UFOMI_CHECK_LAUNCH();
         const ConvP &a = n->dec1[l], &b = n->dec2[l];
         if ((rc = conv3(n, s, cv(n->cat[l], 2 * C), np, l, 2 * C, C, n->w16 + a.w, n->master + a.b, true,
                         cv(nullptr, 0), 0, mv(n->d1[l], C))))

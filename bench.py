@@ -44,6 +44,7 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, os.path.join(ROOT, "ufo-filters_amd"))
 
 MI355X_HBM_TBPS = 8.0
+MI355X_MFMA_TFLOPS = 2500.0  # dense f16 / bf16
 
 
 def log(msg):
@@ -218,8 +219,16 @@ def fbp_parallel(args, ctx, torch, np, ufomi, S, W, P, filt_name, noise, storage
     updates = float(S) * W * W * P
     first = storages[0]
 
+    def on_mfma(st):
+        # stacks go to the matrix cores, unless a tile configuration is forced
+        return not args.bp_config and S >= 12 and updates >= (2.5e9 if st == "f16" else 1e9)
+
     def kname(st):
-        # the instance ufomi_bp_parallel picks: slices per tile, angle chunk, half staging
+        # the instance ufomi_bp_parallel picks: slices per workgroup and planes of the samples, or
+        # slices per tile, angle chunk and half staging
+        if on_mfma(st):
+            unit = "2,2,%d,8" if S > 48 else "1,2,%d,4" if S > 16 else "1,1,%d,4"
+            return "bp_mfma_kernel<%s>" % (unit % (2 if st == "f32" else 1))
         sk = 8 if S >= 8 else (4 if S >= 4 else (2 if S >= 2 else 1))
         return "bp_texture_kernel<%d,%d,%s,%s>" % (sk, 8 if sk >= 4 else 16, STORAGE_NAMES[st],
                                                    "true" if st == "f16" and sk >= 4 else "false")
@@ -274,13 +283,17 @@ def fbp_parallel(args, ctx, torch, np, ufomi, S, W, P, filt_name, noise, storage
     if len(storages) > 1:
         extra["storage_variants"] = variants
     r = runs[first]
-    # LDS bytes read per update: (v, d) float pairs, or half pairs with f16 half staging
-    bpu = 4 if "true" in kernel else 8
+    # LDS bytes read per update: (v, d) float pairs, or half pairs with f16 half staging; on the
+    # matrix cores 8 samples of one or two f16 planes for 16 voxels
+    bpu = (2 if first == "f32" else 1) if on_mfma(first) else 4 if "true" in kernel else 8
+    # products of 8 weights and samples each: both high planes, and the low plane of either side
+    # (weights only when the samples fit one plane)
+    mfma = (48 if first == "f32" else 32) if on_mfma(first) else None
     # compulsory HBM bytes of one backprojection launch: the stored filtered sinograms once, the volume once
     hbm_bytes = float(S) * P * W * (4 if first == "f32" else 2) + float(S) * W * W * 4
     return dict(updates=updates, wall=r["wall"], bp_ms=r["bp_ms"], kernel=kernel, bytes_per_update=bpu,
-                hbm_bytes=hbm_bytes, extra=extra, cpu=cpu, accuracy=accuracy, workload=workload,
-                dtype="f32" if first == "f32" else "f32 accumulate, %s storage" % first,
+                mfma_flops_per_update=mfma, hbm_bytes=hbm_bytes, extra=extra, cpu=cpu, accuracy=accuracy,
+                workload=workload, dtype="f32" if first == "f32" else "f32 accumulate, %s storage" % first,
                 config={"slices": S, "angles": P, "detector": W, "fft_size": N, "storage": first, "filter": filt_name},
                 traffic_key="%s %dx%dx%d %s" % (kernel, S, P, W, first),
                 metric="GUPS (voxel*proj/s) for FBP")
@@ -777,7 +790,7 @@ def main():
             "learned_vs_plain": round(r["learned_sps"] / r["plain_sps"], 3),
             # 18.8 TFLOP over 73.4 GB of compulsory traffic is 256 flop/B, below the 312 flop/B at which
             # 2.5 PFLOP/s and 8 TB/s meet: the forward pass is bound by HBM, and its MFMA rate is reported beside it
-            "roofline": dict({"kernel": "U-Net forward (conv3_t8_kernel, gemm_kernel<...,UpFwd> + VALU layers)", "bound": "hbm",
+            "roofline": dict({"kernel": "U-Net forward (conv3_t8_kernel, up_fwd_kernel + VALU layers)", "bound": "hbm",
                               "achieved": round(r["hbm_achieved"] / 1e9, 1), "peak": MI355X_HBM_TBPS * 1e3, "unit": "GB/s",
                               "frac": round(r["hbm_achieved"] / (MI355X_HBM_TBPS * 1e12), 4),
                               "traffic": traffic_for("U-Net forward learned512 batch256")}, **r["extra"]),
@@ -853,6 +866,13 @@ def roofline_of(r, lds_peak, hbm_copy):
         "hbm_compulsory_GBps": round(r["hbm_bytes"] / bp_s / 1e9, 1),
         "hbm_compulsory_frac_of_8TBps": round(r["hbm_bytes"] / bp_s / 8e12, 5),
     }
+    flops = r.get("mfma_flops_per_update")
+    if flops:
+        # stacks on the matrix cores: their issued products against the dense f16 peak
+        roof.update(bound="mfma", achieved=round(gups * flops / 1e12, 1), peak=MI355X_MFMA_TFLOPS, unit="TFLOP/s",
+                    frac=round(gups * flops / 1e12 / MI355X_MFMA_TFLOPS, 4), mfma_flops_per_update=flops,
+                    peak_source="nominal dense f16", lds_gather_GBps=round(achieved / 1e9, 1),
+                    lds_peak_GBps=round(lds_peak / 1e9, 1))
     if traffic:
         roof["hbm_achieved_GBps"] = round(traffic / bp_s / 1e9, 1)
     valu = entry.get("valu_insts_per_update")

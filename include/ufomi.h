@@ -125,7 +125,7 @@ int ufomi_ifft_rows(ufomi_ctx *ctx, const float *d_in, int N, int P, int crop, f
  * transformed axes normalised by their sizes, real part cropped to
  * crop_width x crop_height (0 = no crop) out, [m2][crop_height][crop_width].
  * Powers of two up to 8192 and other sizes up to 4096 (chirp-z) take one
- * LDS pass per transformed axis.  Longer axes run as two passes of a
+ * pass per transformed axis, a line in a workgroup's registers.  Longer axes run as two passes of a
  * four-step split (powers of two up to 2^20 points) or as Bluestein over that
  * split (other sizes up to 2^19): along the rows of 1-D transforms directly,
  * along any axis of 2-D and 3-D transforms after gathering the lines into

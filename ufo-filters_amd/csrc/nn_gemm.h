@@ -9,8 +9,9 @@
 //   bf16x8 load_b(ColB, k)       B[k .. k+7][n]
 //   void k_range(z, &k0, &k1)    the K slice of split index z (grid z)
 //   void store(m, n, float, z)   epilogue for C[m][n]
-// Convolutions (NHWC activations), their data gradients, the 2x2 transposed
-// convolution and the weight gradients are all such operations.
+// Convolutions (NHWC activations) of small images, the transposed convolution's
+// gradients and narrow levels' weight gradients are such operations; the wide
+// layers have kernels of their own below and in nn_wgrad.h.
 //
 // Lane layout of v_mfma_f32_16x16x32_bf16 (wave of 64, r = lane % 16,
 // q = lane / 16): lane supplies A[r][8q .. 8q+7] and B[8q .. 8q+7][r] and

@@ -7,14 +7,14 @@
 //   skip_l = relu(conv3x3(relu(conv3x3(in_l))))               Conv3 GEMMs; in_l = maxpool(skip_{l-1})
 //   bottom = relu(conv3x3(relu(conv3x3(maxpool(skip_2)))))    C_3 = 256
 //   dec_l  = relu(conv3x3(relu(conv3x3([up_l(src) | skip_l]))))   src = bottom or dec_{l+1}
-//   up_l   = 2x2 stride-2 transposed conv C_{l+1} -> C_l (linear) UpFwd GEMM
+//   up_l   = 2x2 stride-2 transposed conv C_{l+1} -> C_l (linear) up_fwd_kernel
 //   out    = img + conv1x1(dec_0, 32 -> 1)                    fp32, in dec_0's conv epilogue (or final_kernel)
 // The concatenation is never copied: up_l and skip_l are written into the two
 // channel halves of one [pixels][2 C_l] buffer.
 //
 // Training: MSE loss, backward through the same GEMM core (data gradients as
 // convolutions with flipped / transposed weight copies, weight gradients as
-// split-K GEMMs over pixels reduced in a fixed order), Adam on FP32 master
+// products over pixels split between workgroups and added in a fixed order), Adam on FP32 master
 // weights, BF16 copies refreshed after every step.
 #include "ufomi_internal.h"
 #include "nn_gemm.h"

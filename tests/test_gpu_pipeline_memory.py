@@ -76,3 +76,18 @@ def test_blocks_over_sizes_and_streams():
             st.synchronize()
             k = 4 * n * shape[0] * shape[1] if len(shape) == 2 else 4 * n
             assert n == m and torch.equal(got[:k], ref[:k])
+
+
+def test_one_pipeline_on_two_contexts():
+    """A pipeline's coefficients serve every context that runs it; its batches are the running one's."""
+    W, P, S = 64, 9, 3
+    x = torch.randn(S, P, W, device="cuda")
+    a, b = (ufomi.Context(0, torch.cuda.current_stream()) for _ in range(2))
+    pl = ufo_tasks.Pipeline(_text(W, "backproject"))
+    want = pl.run(a, x, out_bytes=4 * S * W * W)[0].clone()
+    for ctx in (b, a, b):
+        assert torch.equal(pl.run(ctx, x, out_bytes=4 * S * W * W)[0], want)
+    del pl
+    other = ufo_tasks.Pipeline(_text(W, "backproject"))
+    assert torch.equal(other.run(a, x, out_bytes=4 * S * W * W)[0], want)
+    del other

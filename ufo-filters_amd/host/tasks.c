@@ -513,11 +513,11 @@ int filter_task_coefficients(UfomiTask *t, size_t width, UfomiError *e)
                                        (float) t->v[FLT_CUTOFF].num, (float) t->v[FLT_ORDER].num,
                                        (float) t->v[FLT_TAU].num, (float) t->v[FLT_THETA].num, h);
     if (!rc && p->d_coef) {
-        ufomi_block_free(t->ctx, p->d_coef);
+        ufomi_device_free(t->ctx, p->d_coef);
         p->d_coef = NULL;
     }
     if (!rc)
-        rc = ufomi_block_alloc(t->ctx, width * sizeof(float), (void **) &p->d_coef);
+        rc = ufomi_device_alloc(t->ctx, width * sizeof(float), (void **) &p->d_coef);
     if (!rc)
         rc = ufomi_memcpy(t->ctx, p->d_coef, h, width * sizeof(float), 0);
     free(h);
@@ -550,7 +550,7 @@ static void filter_finalize(UfomiTask *t)
 {
     FilterPriv *p = t->priv;
     if (p && p->d_coef && t->ctx)
-        ufomi_block_free(t->ctx, p->d_coef);
+        ufomi_device_free(t->ctx, p->d_coef);
 }
 
 /* ----------------------------------------------------------- backproject */

@@ -174,8 +174,12 @@ void ufomi_bp_params_init(ufomi_bp_params *p);
  * weight): 0 or positive = on (the default), negative = off.  Slices and
  * chunk do not change results; half staging does.  With both automatic,
  * stacks of 12 and more slices with enough work run on the matrix cores
- * (two-term f16 samples and weights, f32 sums, 22-bit samples: the same result
- * up to rounding), which asks for no configuration.  No counterpart in the
+ * (two-term f16 samples and weights, f32 sums), which asks for no
+ * configuration: the same result up to rounding.  Samples keep 22 bits there
+ * down to 2^-17 of their slice's largest |sample| and an absolute 2^-40 of it
+ * below; slices of a larger range (more than 1 / 64 of the non-zero samples
+ * below 2^-17), or with an Inf or a NaN, stay off the matrix cores together
+ * with up to 63 neighbours.  No counterpart in the
  * reference.
  */
 int ufomi_bp_configure(ufomi_ctx *ctx, int slices_per_tile, int angle_chunk, int half_staging);

@@ -124,6 +124,32 @@ def test_scales(ctx, torch_dev):
             assert np.abs(got[s] - ref[s]).max() < 400 * 1.5e-45, v
 
 
+@pytest.mark.parametrize("storage,hot", [("f32", 1e8), ("f32", 1e20), ("f32", 3e38), ("bf16", 1e14), ("f16", 65504.0)])
+def test_large_sample_stays_local(ctx, torch_dev, storage, hot):
+    """One large finite sample (angle 0, first detector entry) reaches the first column of voxels and leaves the
+    precision of the others, in its slice and in its neighbours, as the interpolating kernel has it.  f16 storage
+    holds denormals beside its largest value."""
+    x = _stack(torch_dev, 33, 300, 512, storage, seed=11)
+    if storage == "f16":
+        x *= 2.0 ** -20
+    x[5, 0, 0] = hot
+    x[32, 0, 0] = -hot
+    got, ref = (t[:, :, 2:].double().cpu().numpy() for t in _both(ctx, torch_dev, x, storage))
+    for s in range(33):
+        assert rel_l2(got[s], ref[s]) < 1e-5, s
+
+
+def test_small_part_beside_large(ctx, torch_dev):
+    """Voxels that see only the quarter of the detector with samples of order 1, beside 1e12 elsewhere (angles
+    up to 0.4, so the left edge of the upper half stays on that quarter)."""
+    W = 512
+    x = _stack(torch_dev, 16, 400, W, seed=12)
+    x[3, :, W // 4:] *= 1e12
+    got, ref = (t[:, :W // 2, :W // 8].double().cpu().numpy() for t in _both(ctx, torch_dev, x, angle_step=0.001))
+    for s in range(16):
+        assert rel_l2(got[s], ref[s]) < 1e-5, s
+
+
 def test_streams_share_a_context(ctx, torch_dev):
     """Calls of one context on two streams in turn: the second waits for the first one's workspace."""
     import torch

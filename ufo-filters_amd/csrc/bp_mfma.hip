@@ -14,7 +14,14 @@
 // absolute floor of 2^-40 of the slice's maximum); a weight is a multiple of
 // 2^-11 plus a remainder of at most 2^-12 in f16 (to 2^-24).  Three products
 // (l w_h, h w_l, h w_h) leave out only l w_l, 2^-23 of the term.  f16 storage
-// needs no l plane and two products; bf16 storage likewise (8 significant bits).
+// needs no l plane and two products; bf16 storage likewise (8 significant bits
+// down to 2^-32 of the slice's maximum).
+//
+// The floor is absolute, so one large sample would take the precision of its
+// whole slice.  A slice of which more than 1 / 64 of the non-zero samples lie
+// below kSmall (where the floor leaves fewer bits than stated above) is left to
+// the interpolating kernel with its unit, as is one that holds an Inf or a NaN.
+// Noise puts 2e-5 of the samples there.
 #include "ufomi_internal.h"
 
 #include <algorithm>
@@ -29,6 +36,12 @@ constexpr int kSub = 32;     // slices per stored row
 constexpr int kRow = kSub * 2;             // bytes of one plane's row of one detector entry
 constexpr int kPlane = kSpan * kRow;       // bytes of one staged plane of one angle
 constexpr int kParChunk = 64;              // angles per parameter chunk
+// Scaled samples below this keep fewer than 22 bits (f32 storage), 8 bits (bf16); f16 ones are exact.
+template <typename T> constexpr float kSmall = 0.125f;
+template <> constexpr float kSmall<__hip_bfloat16> = 0x1p-17f;
+template <> constexpr float kSmall<__half> = 0.0f;
+constexpr unsigned kSmallShare = 64;
+constexpr unsigned kLeftOut = 0x7f800000u;  // from here on, a slice's word of maxbits leaves its unit out
 // Row workspace of a call: as many groups as fit, one at least; a larger group takes the other path.
 constexpr size_t kWorkspace = (size_t) 1 << 30, kGroupMax = (size_t) 4 << 30;
 
@@ -49,44 +62,62 @@ __global__ __launch_bounds__(256) void clear_kernel(unsigned *__restrict__ p, in
 }
 
 // Largest |v| of every slice, as the bits of a float: ordered like the value, Inf and NaN above all.
+// Also the number of its non-zero samples.
 template <typename T>
 __global__ __launch_bounds__(256) void absmax_kernel(const T *__restrict__ sino, long pitch, long n,
-                                                     unsigned *__restrict__ maxbits)
+                                                     unsigned *__restrict__ maxbits, unsigned *__restrict__ nonzero)
 {
     const T *s = sino + (long) blockIdx.y * pitch;
     const long step = (long) gridDim.x * 256;
-    unsigned m = 0;
+    unsigned m = 0, c = 0;
+    auto add = [&](T v) {
+        const unsigned bits = __float_as_uint(to_float(v)) & 0x7fffffffu;
+        m = max(m, bits);
+        c += bits != 0;
+    };
     long i = (long) blockIdx.x * 256 + threadIdx.x;
     for (; i + 7 * step < n; i += 8 * step) {
         T v[8];
 #pragma unroll
         for (int k = 0; k < 8; k++) v[k] = s[i + k * step];
 #pragma unroll
-        for (int k = 0; k < 8; k++) m = max(m, __float_as_uint(to_float(v[k])) & 0x7fffffffu);
+        for (int k = 0; k < 8; k++) add(v[k]);
     }
-    for (; i < n; i += step) m = max(m, __float_as_uint(to_float(s[i])) & 0x7fffffffu);
+    for (; i < n; i += step) add(s[i]);
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) m = max(m, (unsigned) __shfl_xor((int) m, o, 64));
-    __shared__ unsigned red[4];
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
+    for (int o = 32; o > 0; o >>= 1) {
+        m = max(m, (unsigned) __shfl_xor((int) m, o, 64));
+        c += (unsigned) __shfl_xor((int) c, o, 64);
+    }
+    __shared__ unsigned red[4], cnt[4];
+    if ((threadIdx.x & 63) == 0) {
+        red[threadIdx.x >> 6] = m;
+        cnt[threadIdx.x >> 6] = c;
+    }
     __syncthreads();
-    if (threadIdx.x == 0)
+    if (threadIdx.x == 0) {
         atomicMax(maxbits + blockIdx.y, max(max(red[0], red[1]), max(red[2], red[3])));
+        atomicAdd(nonzero + blockIdx.y, cnt[0] + cnt[1] + cnt[2] + cnt[3]);
+    }
 }
 
-// Power of two that takes the slice's maximum into [2^14, 2^15).
-__device__ __forceinline__ int scale_exponent(unsigned maxbits)
+// Power of two that takes the slice's maximum into [2^14, 2^15), or for one plane, whose samples
+// have at most 11 bits, into [2^15, 2^16): f16 storage is never scaled down, and so exact.
+template <int PL> __device__ __forceinline__ int scale_exponent(unsigned maxbits)
 {
-    if (maxbits == 0 || maxbits >= 0x7f800000u) return 0;
-    return min(14 + 127 - (int) (maxbits >> 23), 126);
+    if (maxbits == 0 || maxbits >= kLeftOut) return 0;
+    return min(16 - PL + 127 - (int) (maxbits >> 23), 126);
 }
 
 // Scaled and split rows, slices innermost: ws[group][angle][plane][detector entry][32 slices] f16,
 // kPad zero entries on both sides, zero rows up to a multiple of 4 angles.  The two halves of a
-// row swap places at odd angles (the bank layout of the tile kernel's reads).
+// row swap places at odd angles (the bank layout of the tile kernel's reads).  Counts the small
+// samples of a slice and marks it in maxbits when they are too many; what its rows hold from then
+// on is not used.
 template <typename T, int PL>
 __global__ __launch_bounds__(256) void split_kernel(const T *__restrict__ sino, long pitch, int W, int P, int Wp,
-                                                    int n_slices, const unsigned *__restrict__ maxbits,
+                                                    int n_slices, unsigned *maxbits,
+                                                    const unsigned *__restrict__ nonzero, unsigned *small,
                                                     uint4_t *__restrict__ ws, long group_stride)
 {
     constexpr int PITCH = kSub / 2 + 1;  // dwords per entry in LDS
@@ -101,13 +132,18 @@ __global__ __launch_bounds__(256) void split_kernel(const T *__restrict__ sino, 
         const int s = g * kSub + wv * 8 + k;
         v[k] = in && s < n_slices ? to_float(sino[(long) s * pitch + (long) p * W + j]) : 0.0f;
     }
+    unsigned few = 0;  // small samples of slice wv * 8 + lane, lane < 8
 #pragma unroll
     for (int k = 0; k < 8; k += 2) {
         unsigned hp = 0, lp = 0;
 #pragma unroll
         for (int q = 0; q < 2; q++) {
             const int s = g * kSub + wv * 8 + k + q;
-            const float x = ldexpf(v[k + q], scale_exponent(maxbits[min(s, n_slices - 1)]));
+            const float x = ldexpf(v[k + q], scale_exponent<PL>(maxbits[min(s, n_slices - 1)]));
+            if constexpr (kSmall<T> > 0.0f) {
+                const unsigned c = __popcll(__ballot(v[k + q] != 0.0f && fabsf(x) < kSmall<T>));
+                if (lane == k + q) few = c;
+            }
             const _Float16 h = (_Float16) x;
             hp |= (unsigned) __builtin_bit_cast(unsigned short, h) << (16 * q);
             if constexpr (PL == 2) {
@@ -117,6 +153,15 @@ __global__ __launch_bounds__(256) void split_kernel(const T *__restrict__ sino, 
         }
         tile[0][lane * PITCH + wv * 4 + k / 2] = hp;
         if constexpr (PL == 2) tile[PL - 1][lane * PITCH + wv * 4 + k / 2] = lp;
+    }
+    if constexpr (kSmall<T> > 0.0f) {
+        // a slice that is marked already (read past the caches) is not counted on: its counter
+        // would be all that the waves wait for
+        const int s = g * kSub + wv * 8 + lane;  // < n_slices where few > 0: the padding is zeros
+        if (few && __hip_atomic_load(maxbits + s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < kLeftOut) {
+            const unsigned limit = nonzero[s] / kSmallShare, before = atomicAdd(small + s, few);
+            if (before <= limit && before + few > limit) atomicMax(maxbits + s, kLeftOut);
+        }
     }
     __syncthreads();
     const int e = threadIdx.x >> 2, part = threadIdx.x & 3;
@@ -211,9 +256,10 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NT == 1
     const int band_h = min(8, tiles_y - 8 * band);
     const int ty = 8 * band + in_band % band_h, tx = in_band / band_h;
     const int slice0 = unit * UNIT;
-    // a slice that holds an Inf or a NaN would spread it over a block: such a unit is left to
-    // the interpolating kernel, which runs after this one
-    if (__ballot(maxbits[min(slice0 + min(lane, UNIT - 1), n_slices - 1)] >= 0x7f800000u)) return;
+    // a slice that holds an Inf or a NaN would spread it over a block, and one of too many small
+    // samples would lose them: such a unit is left to the interpolating kernel, which runs after
+    // this one
+    if (__ballot(maxbits[min(slice0 + min(lane, UNIT - 1), n_slices - 1)] >= kLeftOut)) return;
     const int p0 = (int) blockIdx.y * p_chunk;
     const int np = min(p_chunk, P - p0);
     const int nq = (np + 3) >> 2;
@@ -406,7 +452,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NT == 1
 #pragma unroll
     for (int n = 0; n < NG * NT; n++) {
         const int sl = slice0 + (n / NT) * kSub + (n % NT) * 16 + l16;
-        const float inv = sl < n_slices ? ldexpf(1.0f, -scale_exponent(maxbits[sl])) : 0.0f;
+        const float inv = sl < n_slices ? ldexpf(1.0f, -scale_exponent<PL>(maxbits[sl])) : 0.0f;
 #pragma unroll
         for (int i = 0; i < BPW; i++) {
             const int x = x0 + 4 * ((wb + i) & 7), y = y0 + 4 * ((wb + i) >> 3) + g;
@@ -516,14 +562,16 @@ template <typename T, int PL> int run(ufomi_ctx *ctx, const T *sino, const ufomi
     const int P4 = (st.P + 3) / 4 * 4;
     const int p_chunk = n_split > 1 ? (P4 / 4 + n_split - 1) / n_split * 4 : P4;
     n_split = (P4 + p_chunk - 1) / p_chunk;
-    const size_t head = ((size_t) per_chunk * kSub * sizeof(unsigned) + 255) & ~(size_t) 255;
+    // per slice: largest |v|, number of non-zero and of small samples
+    const int words = per_chunk * kSub;
+    const size_t head = (3 * (size_t) words * sizeof(unsigned) + 255) & ~(size_t) 255;
     const size_t rows_bytes = gb * per_chunk;
     const size_t part_bytes =
         n_split > 1 ? (size_t) n_split * std::min(per_chunk * kSub, n_slices) * plane * sizeof(float) : 0;
     int rc = acquire_workspace(ctx, head + rows_bytes + part_bytes);
     if (rc == UFOMI_ERR_MEMORY) return UFOMI_OK;  // *done = 0
     if (rc) return rc;
-    unsigned *maxbits = (unsigned *) ctx->ws;
+    unsigned *maxbits = (unsigned *) ctx->ws, *nonzero = maxbits + words, *small = nonzero + words;
     char *rows = (char *) ctx->ws + head;
     float *part = n_split > 1 ? (float *) (rows + rows_bytes) : nullptr;
     const int Wp = st.W + 2 * kPad;
@@ -533,14 +581,16 @@ template <typename T, int PL> int run(ufomi_ctx *ctx, const T *sino, const ufomi
         const int ng = (ns + kSub - 1) / kSub;
         const T *in = sino + (size_t) s0 * st.sino_pitch;
         float *out = st.out + (size_t) s0 * st.out_pitch;
-        hipLaunchKernelGGL(clear_kernel, dim3((ns + 255) / 256), dim3(256), 0, ctx->stream, maxbits, ns);
+        hipLaunchKernelGGL(clear_kernel, dim3((3 * words + 255) / 256), dim3(256), 0, ctx->stream, maxbits,
+                           3 * words);
         UFOMI_CHECK_LAUNCH();
         const unsigned mb = (unsigned) std::min<long>((elems + 8191) / 8192, 64);
         hipLaunchKernelGGL(absmax_kernel<T>, dim3(mb, ns), dim3(256), 0, ctx->stream, in, (long) st.sino_pitch, elems,
-                           maxbits);
+                           maxbits, nonzero);
         UFOMI_CHECK_LAUNCH();
         hipLaunchKernelGGL((split_kernel<T, PL>), dim3((Wp + 63) / 64, P4, ng), dim3(256), 0, ctx->stream, in,
-                           (long) st.sino_pitch, st.W, st.P, Wp, ns, maxbits, (uint4_t *) rows, (long) (gb / 16));
+                           (long) st.sino_pitch, st.W, st.P, Wp, ns, maxbits, nonzero, small, (uint4_t *) rows,
+                           (long) (gb / 16));
         UFOMI_CHECK_LAUNCH();
         // `count` slices from slice `first` of the chunk, `unit` per workgroup
         auto launch = [&](auto kernel, int threads, int unit, int first, int count) {
@@ -566,7 +616,7 @@ template <typename T, int PL> int run(ufomi_ctx *ctx, const T *sino, const ufomi
                                0, ctx->stream, part, n_split, total, plane, out, (long) st.out_pitch);
             UFOMI_CHECK_LAUNCH();
         }
-        if ((rc = ufomi_bp_nonfinite(ctx, st, s0, ns, a, b, maxbits))) return rc;
+        if ((rc = ufomi_bp_left_out(ctx, st, s0, ns, a, b, maxbits))) return rc;
     }
     UFOMI_HIP(hipEventRecord(ctx->ws_event, ctx->stream));
     *done = n_slices;

@@ -119,10 +119,10 @@ struct ufomi_bp_stack {
 };
 // Backprojects the first *done slices (0: none, the caller's other path takes all of them).
 int ufomi_bp_mfma(ufomi_ctx *ctx, const ufomi_bp_stack &st, int *done);
-// Slices s0 .. s0 + ns - 1 again where a unit that holds an Inf or a NaN (maxbits) was left out:
+// Those of slices s0 .. s0 + ns - 1 whose unit was left out (a word of maxbits of 0x7f800000 or more):
 // units of 64 slices up to n64, of 32 up to n32, of 16 after.
-int ufomi_bp_nonfinite(ufomi_ctx *ctx, const ufomi_bp_stack &st, int s0, int ns, int n64, int n32,
-                       const unsigned *maxbits);
+int ufomi_bp_left_out(ufomi_ctx *ctx, const ufomi_bp_stack &st, int s0, int ns, int n64, int n32,
+                      const unsigned *maxbits);
 
 // Takes the calling thread's current device's address of the preallocated
 // scratch of ufomi_bp_parallel_noalloc (once per device; ufomi_create).

@@ -92,6 +92,29 @@ def test_geometry_and_pitches(ctx, torch_dev, props):
     np.testing.assert_array_equal(flat[0][:, :rw * rh].reshape(S, rh, rw), got.cpu().numpy())
 
 
+@pytest.mark.parametrize("S,P,W,roi,matrix", [
+    (12, 65532, 16, 36, True),     # the largest angle count, rounded up to fours, of the layout's grid
+    (12, 65533, 16, 36, False),
+    (12, 70001, 16, 36, False),
+    (65504, 16, 8, 32, True),      # the most slices of one chunk
+    (65600, 16, 8, 32, True),      # and the first that take two
+])
+def test_launch_limits(ctx, torch_dev, S, P, W, roi, matrix):
+    """A grid's second axis holds 65535 blocks: more slices go in chunks, more angles to the interpolating kernel."""
+    import torch
+    x = _stack(torch_dev, S, P, W, seed=13)
+    got, ref = _both(ctx, torch_dev, x, roi_width=roi, roi_height=roi)
+    assert torch.equal(got, ref) != matrix
+    assert bool(torch.isfinite(got).all())
+    err = (got - ref).double().norm(dim=(1, 2)) / ref.double().norm(dim=(1, 2))
+    # float32 sums of P terms of order 1: both round at up to 2^-24 of the partial sums, whose size is that of
+    # the result (a random walk) -> P^0.5 roundings
+    assert float(err.max()) < 1e-5 + 2.0 ** -24 * P ** 0.5
+    if not matrix or S < 100:
+        exact = oracle.bp_texture_f64(x[S // 2].cpu().numpy(), axis_pos=W / 2.0, roi_width=roi, roi_height=roi)
+        assert rel_l2(got[S // 2].cpu().numpy(), exact) < 1e-5 + 2.0 ** -24 * P ** 0.5
+
+
 @pytest.mark.parametrize("storage", ["f32", "f16", "bf16"])
 def test_nonfinite_values_stay_local(ctx, torch_dev, storage):
     """An Inf or a NaN reaches the pixels whose samples touch it and no others, whichever unit it is in."""

@@ -42,6 +42,7 @@ template <> constexpr float kSmall<__hip_bfloat16> = 0x1p-17f;
 template <> constexpr float kSmall<__half> = 0.0f;
 constexpr unsigned kSmallShare = 64;
 constexpr unsigned kLeftOut = 0x7f800000u;  // from here on, a slice's word of maxbits leaves its unit out
+constexpr int kGridY = 65535;  // a grid's second axis: the angles of split_kernel, the slices of absmax_kernel
 // Row workspace of a call: as many groups as fit, one at least; a larger group takes the other path.
 constexpr size_t kWorkspace = (size_t) 1 << 30, kGroupMax = (size_t) 4 << 30;
 
@@ -550,7 +551,7 @@ template <typename T, int PL> int run(ufomi_ctx *ctx, const T *sino, const ufomi
     const size_t gb = group_bytes(st.W, st.P, PL);
     const int groups_all = (n_slices + kSub - 1) / kSub;
     // whole units of 64 slices per chunk, unless one does not fit
-    int per_chunk = (int) std::max<size_t>(1, std::min<size_t>(kWorkspace / gb, (size_t) groups_all));
+    int per_chunk = (int) std::max<size_t>(1, std::min<size_t>({kWorkspace / gb, (size_t) groups_all, kGridY / kSub}));
     if (per_chunk > 1 && per_chunk < groups_all) per_chunk &= ~1;
     const int tiles_x = (st.roi_w + kTile - 1) / kTile, tiles_y = (st.roi_h + kTile - 1) / kTile;
     const long tiles = (long) tiles_x * tiles_y, plane = (long) st.roi_w * st.roi_h;
@@ -632,7 +633,7 @@ int ufomi_bp_mfma(ufomi_ctx *ctx, const ufomi_bp_stack &st, int *done)
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     UFOMI_HIP(hipStreamIsCapturing(ctx->stream, &cap));
     if (cap != hipStreamCaptureStatusNone) return UFOMI_OK;
-    if (group_bytes(st.W, st.P, st.dtype == UFOMI_F32 ? 2 : 1) > kGroupMax) return UFOMI_OK;
+    if (group_bytes(st.W, st.P, st.dtype == UFOMI_F32 ? 2 : 1) > kGroupMax || st.P > kGridY / 4 * 4) return UFOMI_OK;
     const long tiles = (long) ((st.roi_w + kTile - 1) / kTile) * ((st.roi_h + kTile - 1) / kTile);
     if (tiles * ((st.n_slices + 15) / 16) > 0x7fffffffL) return UFOMI_OK;
     switch (st.dtype) {

@@ -174,12 +174,13 @@ def test_small_part_beside_large(ctx, torch_dev):
 
 
 def test_streams_share_a_context(ctx, torch_dev):
-    """Calls of one context on two streams in turn: the second waits for the first one's workspace."""
+    """Calls of one context on two streams in turn: the second waits for the first one's workspace.  Both have
+    the same angles, whose table stays as it is (a new one frees the last, which waits for every stream)."""
     import torch
-    a, b = _stack(torch_dev, 64, 400, 512, seed=1), _stack(torch_dev, 48, 300, 400, seed=2)
+    a, b = _stack(torch_dev, 64, 400, 512, seed=1), _stack(torch_dev, 48, 400, 400, seed=2)
     oa, ob = torch.empty((64, 512, 512), device=torch_dev), torch.empty((48, 400, 400), device=torch_dev)
     ctx.bp_parallel(a, 512, 400, oa, n_slices=64)
-    ctx.bp_parallel(b, 400, 300, ob, n_slices=48)
+    ctx.bp_parallel(b, 400, 400, ob, n_slices=48)
     torch.cuda.synchronize()
     ra, rb = oa.clone(), ob.clone()
     side = torch.cuda.Stream()
@@ -188,12 +189,13 @@ def test_streams_share_a_context(ctx, torch_dev):
     try:
         for _ in range(4):
             oa.zero_()
+            ob.zero_()
+            torch.cuda.synchronize()
             ctx.set_stream(main)
             ctx.bp_parallel(a, 512, 400, oa, n_slices=64)
             ctx.set_stream(side)
             with torch.cuda.stream(side):
-                ob.zero_()
-                ctx.bp_parallel(b, 400, 300, ob, n_slices=48)
+                ctx.bp_parallel(b, 400, 400, ob, n_slices=48)
             torch.cuda.synchronize()
             assert torch.equal(oa, ra) and torch.equal(ob, rb)
     finally:

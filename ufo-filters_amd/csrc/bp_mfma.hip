@@ -491,8 +491,9 @@ size_t group_bytes(int W, int P, int planes)
     return (size_t) ((P + 3) / 4 * 4) * planes * (W + 2 * kPad) * kRow;
 }
 
-// The row workspace is shared by all calls of a context: a call on another stream than the
-// last one's waits for it.
+// The row workspace is shared by all calls of a context: a call waits for the last one's event,
+// whatever stream that was on (on the same one the wait is free, and a new stream may have the
+// handle of one that was destroyed with work pending).
 int acquire_workspace(ufomi_ctx *ctx, size_t bytes)
 {
     if (!ctx->ws_event)
@@ -510,10 +511,9 @@ int acquire_workspace(ufomi_ctx *ctx, size_t bytes)
             return UFOMI_ERR_MEMORY;
         }
         ctx->ws_bytes = bytes;
-    } else if (ctx->ws_stream != ctx->stream) {
+    } else {
         UFOMI_HIP(hipStreamWaitEvent(ctx->stream, ctx->ws_event, 0));
     }
-    ctx->ws_stream = ctx->stream;
     return UFOMI_OK;
 }
 
@@ -577,7 +577,7 @@ template <typename T, int PL> int run(ufomi_ctx *ctx, const T *sino, const ufomi
     float *part = n_split > 1 ? (float *) (rows + rows_bytes) : nullptr;
     const int Wp = st.W + 2 * kPad;
     const long elems = (long) st.P * st.W;
-    for (int g0 = 0; g0 < groups_all; g0 += per_chunk) {
+    auto chunk = [&](int g0) {
         const int s0 = g0 * kSub, ns = std::min(per_chunk * kSub, n_slices - s0);
         const int ng = (ns + kSub - 1) / kSub;
         const T *in = sino + (size_t) s0 * st.sino_pitch;
@@ -608,20 +608,22 @@ template <typename T, int PL> int run(ufomi_ctx *ctx, const T *sino, const ufomi
         };
         const Units u = units_of(ns);
         const int a = std::min(64 * u.n64, ns), b = std::min(a + 32 * u.n32, ns), e = std::min(b + 16 * u.n16, ns);
-        if ((rc = launch(bp_mfma_kernel<2, 2, PL, 8>, 512, 64, 0, a))) return rc;
-        if ((rc = launch(bp_mfma_kernel<1, 2, PL, 4>, 256, 32, a, b - a))) return rc;
-        if ((rc = launch(bp_mfma_kernel<1, 1, PL, 4>, 256, 16, b, e - b))) return rc;
+        if (int rc = launch(bp_mfma_kernel<2, 2, PL, 8>, 512, 64, 0, a)) return rc;
+        if (int rc = launch(bp_mfma_kernel<1, 2, PL, 4>, 256, 32, a, b - a)) return rc;
+        if (int rc = launch(bp_mfma_kernel<1, 1, PL, 4>, 256, 16, b, e - b)) return rc;
         if (part) {
             const long total = plane * ns;
             hipLaunchKernelGGL(sum_parts_kernel, dim3((unsigned) std::min<long>((total + 255) / 256, 8192)), dim3(256),
                                0, ctx->stream, part, n_split, total, plane, out, (long) st.out_pitch);
             UFOMI_CHECK_LAUNCH();
         }
-        if ((rc = ufomi_bp_left_out(ctx, st, s0, ns, a, b, maxbits))) return rc;
-    }
+        return ufomi_bp_left_out(ctx, st, s0, ns, a, b, maxbits);
+    };
+    for (int g0 = 0; g0 < groups_all && !rc; g0 += per_chunk) rc = chunk(g0);
+    // also where a launch failed: those before it use the workspace
     UFOMI_HIP(hipEventRecord(ctx->ws_event, ctx->stream));
-    *done = n_slices;
-    return UFOMI_OK;
+    if (!rc) *done = n_slices;
+    return rc;
 }
 
 }  // namespace

@@ -46,12 +46,10 @@ struct ufomi_ctx {
     // partial sums of angle-split backprojections of few tiles (grow-only)
     float *bp_part;
     size_t bp_part_bytes;
-    // row workspace of stack backprojections (bp_mfma.hip, grow-only), the event of its last
-    // use and the stream of that use
+    // row workspace of stack backprojections (bp_mfma.hip, grow-only) and the event of its last use
     void *ws;
     size_t ws_bytes;
     hipEvent_t ws_event;
-    hipStream_t ws_stream;
     ufomi_chirp chirps[8];   // the last used Bluestein tables (at most 96 KiB each)
     unsigned long chirp_clock;
     ufomi_block blocks[8];   // at most 512 MiB in all, busy ones included

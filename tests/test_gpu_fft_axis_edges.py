@@ -40,8 +40,66 @@ def test_line_lengths(ctx, torch_dev, axis, m):
 def test_tables_of_many_sizes(ctx, torch_dev):
     """More sizes in turn than the context keeps Bluestein tables for, and back to the first."""
     import torch
-    for m in list(range(90, 110)) + [90, 95]:
+    for m in list(range(90, 160)) + [90, 95]:
         x = np.random.default_rng(m).standard_normal((4, m, m + 1)).astype(np.float32)
         spec = torch.empty((4, m, m + 1, 2), device=torch_dev)
         ctx.fft_nd(torch.from_numpy(x).to(torch_dev), (m + 1, m, 4), 2, (m + 1, m, 4), spec)
         assert rel_l2(torch.view_as_complex(spec).cpu().numpy(), np.fft.fft2(x.astype(np.float64))) < 1e-6
+
+
+def test_streams_with_many_sizes(torch_dev):
+    """More tables than the context keeps, used on two streams in turn: one is replaced only when no stream
+    reads it any more."""
+    import torch
+    import ufomi
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    c = ufomi.Context(0, streams[0])
+    held = []
+    for i, m in enumerate(list(range(300, 370)) + [300, 301]):
+        st = streams[i % 2]
+        c.set_stream(st)
+        with torch.cuda.stream(st):
+            x = torch.randn((40, m, m), device=torch_dev)
+            spec = torch.empty((40, m, m, 2), device=torch_dev)
+            c.fft_nd(x, (m, m, 40), 2, (m, m, 40), spec)
+            held.append((x, spec))
+    torch.cuda.synchronize()
+    for x, spec in held:
+        ref = np.fft.fft2(x[7].cpu().numpy().astype(np.float64))
+        assert rel_l2(torch.view_as_complex(spec[7]).cpu().numpy(), ref) < 1e-6
+    c.close()
+
+
+def test_capture(torch_dev):
+    """A transform with tables is refused under capture, first call or not; one without is captured."""
+    import torch
+    import ufomi
+    st = torch.cuda.Stream()
+    c = ufomi.Context(0, st)
+    for m in (96, 100):
+        x = torch.randn((3, 64, m), device=torch_dev)
+        spec = torch.zeros((3, 64, m, 2), device=torch_dev)
+        torch.cuda.synchronize()
+        for known in (False, True):
+            g = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(g, stream=st):
+                spec.zero_()
+                with pytest.raises(ufomi.UfomiError):
+                    c.fft_nd(x, (m, 64, 3), 2, (m, 64, 3), spec)
+            if not known:
+                c.fft_nd(x, (m, 64, 3), 2, (m, 64, 3), spec)
+                torch.cuda.synchronize()
+                assert rel_l2(torch.view_as_complex(spec).cpu().numpy(), np.fft.fft2(x.double().cpu().numpy())) < 1e-6
+    x, spec = torch.randn((3, 64, 128), device=torch_dev), torch.zeros((3, 64, 128, 2), device=torch_dev)
+    c.fft_nd(x, (128, 64, 3), 2, (128, 64, 3), spec)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=st):
+        c.fft_nd(x, (128, 64, 3), 2, (128, 64, 3), spec)
+    for k in range(3):
+        x.normal_()
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        assert rel_l2(torch.view_as_complex(spec).cpu().numpy(), np.fft.fft2(x.double().cpu().numpy())) < 1e-6
+    c.close()

@@ -121,6 +121,7 @@ extern "C" int ufomi_create(int device, ufomi_ctx **out)
     ufomi_ctx *ctx = (ufomi_ctx *) calloc(1, sizeof(ufomi_ctx));
     ctx->device = device;
     ctx->stream = nullptr;
+    ctx->stream_epoch = 1;
 
     // Twiddles exp(-2 pi i k / M), evaluated in FP64 and rounded once to float.
     const int M = UFOMI_FFT_MAX;
@@ -185,9 +186,8 @@ extern "C" int ufomi_destroy(ufomi_ctx *ctx)
     }
     if (ctx->ws_event)
         (void) hipEventDestroy(ctx->ws_event);
-    for (ufomi_chirp &c : ctx->chirps)
-        if (c.table)
-            (void) hipFree(c.table);
+    if (ctx->chirp_mem)
+        (void) hipFree(ctx->chirp_mem);
     trim_blocks(ctx);
     if (ctx->scratch)
         (void) hipFree(ctx->scratch);
@@ -202,6 +202,7 @@ extern "C" int ufomi_set_stream(ufomi_ctx *ctx, void *stream)
     if (!ctx)
         return ufomi_fail(UFOMI_ERR_ARG, "null context");
     ctx->stream = (hipStream_t) stream;
+    ctx->stream_epoch++;
     return UFOMI_OK;
 }
 

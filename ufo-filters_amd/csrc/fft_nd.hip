@@ -370,40 +370,66 @@ int launch_pass(hipStream_t s, const PassSpec &ps, const void *in, void *out, co
     return UFOMI_OK;
 }
 
-// The Bluestein tables of M points, from the context's few last used ones: they depend on the size
-// and direction alone, and forming them takes the host about a millisecond at 2048 points.
-int chirp_tables(ufomi_ctx *ctx, int M, int L, int dir, const float2 **out)
+// The Bluestein tables of every pass, from the context's last used ones: they depend on the size
+// and direction alone, and forming them takes the host about a millisecond at 2048 points.  64 of
+// them hold a forward and back of ten 3-D sizes; another one takes the place of the one used
+// longest ago (2-D transforms of 300 to 340 points there and back: 38 us with kept tables, 378 us
+// where each is formed again, 346 us with tables formed for every call into the scratch memory).
+int chirp_tables(ufomi_ctx *ctx, PassSpec *ps, int np, int dir)
 {
-    ufomi_chirp *slot = &ctx->chirps[0];
-    for (ufomi_chirp &c : ctx->chirps) {
-        if (c.table && c.M == M && c.dir == dir) {
-            c.used = ++ctx->chirp_clock;
-            *out = c.table;
-            return UFOMI_OK;
+    if (!ctx->chirp_mem)
+        UFOMI_HIP(ufomi_malloc(ctx, (void **) &ctx->chirp_mem, kChirps * kChirpElems * sizeof(float2)));
+    std::vector<float2> h[3];
+    ufomi_chirp *slots[3] = {};
+    bool others = false;
+    int missing = 0;
+    for (int p = 0; p < np; p++) {
+        if (!ps[p].chirp) continue;
+        const int M = ps[p].M, L = ps[p].g.L;
+        ufomi_chirp *slot = nullptr, *oldest = &ctx->chirps[0];
+        for (ufomi_chirp &c : ctx->chirps) {
+            if (c.M == M && c.dir == dir) slot = &c;
+            if (c.used < oldest->used) oldest = &c;
         }
-        if (c.used < slot->used) slot = &c;
+        if (!slot) {
+            slot = oldest;
+            others |= slot->M && slot->epoch != ctx->stream_epoch;
+            h[p].resize((size_t) M + L);
+            bluestein_tables(M, L, dir, h[p].data(), h[p].data() + M);
+            *slot = ufomi_chirp{M, dir, 0, ctx->stream_epoch};
+            slots[p] = slot;
+            missing++;
+        }
+        slot->used = ++ctx->chirp_clock;
+        if (slot->epoch != ctx->stream_epoch) slot->epoch = 0;
+        ps[p].tables = ctx->chirp_mem + (slot - ctx->chirps) * kChirpElems;
     }
-    std::vector<float2> h((size_t) M + L);
-    bluestein_tables(M, L, dir, h.data(), h.data() + M);
-    if (slot->table) {
-        UFOMI_HIP(hipDeviceSynchronize());  // earlier transforms, on any stream, may still read it
-        UFOMI_HIP(hipFree(slot->table));
-        *slot = ufomi_chirp{};
+    if (!missing) return UFOMI_OK;
+    // earlier transforms may still read the old tables: on this stream or on another one set before
+    hipError_t e = others ? hipDeviceSynchronize() : hipStreamSynchronize(ctx->stream);
+    for (int p = 0; p < np && e == hipSuccess; p++)
+        if (slots[p])
+            e = hipMemcpyAsync((void *) ps[p].tables, h[p].data(), h[p].size() * sizeof(float2), hipMemcpyHostToDevice,
+                               ctx->stream);
+    const hipError_t done = hipStreamSynchronize(ctx->stream);  // the copies read h
+    if (e == hipSuccess) e = done;
+    if (e != hipSuccess) {
+        for (ufomi_chirp *c : slots)
+            if (c) *c = ufomi_chirp{};
+        return ufomi_fail(UFOMI_ERR_HIP, "upload of transform tables failed: %s", hipGetErrorString(e));
     }
-    float2 *t = nullptr;
-    UFOMI_HIP(hipMalloc(&t, h.size() * sizeof(float2)));
-    if (hipMemcpy(t, h.data(), h.size() * sizeof(float2), hipMemcpyHostToDevice) != hipSuccess) {
-        (void) hipFree(t);
-        return ufomi_fail(UFOMI_ERR_HIP, "chirp table upload failed");
-    }
-    *slot = ufomi_chirp{t, M, dir, ++ctx->chirp_clock};
-    *out = t;
     return UFOMI_OK;
 }
 
 // Scratch: two complex intermediates of `tmp_elems`; and the Bluestein tables of every pass.
 int setup_scratch(ufomi_ctx *ctx, PassSpec *ps, int np, int dir, size_t tmp_elems, float2 **tmp0, float2 **tmp1)
 {
+    // refused under capture: a graph would keep the address of a table that others replace
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    for (int p = 0; p < np && cap == hipStreamCaptureStatusNone; p++)
+        if (ps[p].chirp) UFOMI_HIP(hipStreamIsCapturing(ctx->stream, &cap));
+    if (cap != hipStreamCaptureStatusNone)
+        return ufomi_fail(UFOMI_ERR_HIP, "a transform whose size is not a power of two cannot be captured");
     const size_t tmp_bytes = ((tmp_elems * sizeof(float2) + 255) / 256) * 256;
     void *base = nullptr;
     int rc = ufomi_scratch(ctx, 2 * tmp_bytes, &base);
@@ -411,7 +437,7 @@ int setup_scratch(ufomi_ctx *ctx, PassSpec *ps, int np, int dir, size_t tmp_elem
     *tmp0 = (float2 *) base;
     *tmp1 = (float2 *) ((char *) base + tmp_bytes);
     for (int p = 0; p < np; p++)
-        if (ps[p].chirp && (rc = chirp_tables(ctx, ps[p].M, ps[p].g.L, dir, &ps[p].tables))) return rc;
+        if (ps[p].chirp) return chirp_tables(ctx, ps, np, dir);
     return UFOMI_OK;
 }
 

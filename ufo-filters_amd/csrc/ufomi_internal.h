@@ -13,10 +13,12 @@
 
 // Bluestein tables of one transform size and direction (fft_nd.hip): chirp[M], kernel spectrum[L].
 struct ufomi_chirp {
-    float2 *table;
-    int M, dir;
+    int M, dir;              // M = 0: empty
     unsigned long used;
+    unsigned long epoch;     // the context's stream_epoch of all its uses; 0: of several
 };
+constexpr int kChirps = 64;                 // tables a context keeps
+constexpr size_t kChirpElems = 4096 + 8192; // of the longest (float2)
 
 // Device block kept for the batches of pipelines (ufomi_block_alloc).
 struct ufomi_block {
@@ -28,6 +30,7 @@ struct ufomi_block {
 struct ufomi_ctx {
     int device;
     hipStream_t stream;
+    unsigned long stream_epoch;  // counts from 1 the streams set so far
     float2 *twiddles;        // exp(-2 pi i k / UFOMI_FFT_MAX), k < UFOMI_FFT_MAX
     float2 *tw16;            // the same values laid out for the passes of every size (fft16::Tab)
     int *flags;              // small device words written by classification kernels
@@ -50,7 +53,8 @@ struct ufomi_ctx {
     void *ws;
     size_t ws_bytes;
     hipEvent_t ws_event;
-    ufomi_chirp chirps[8];   // the last used Bluestein tables (at most 96 KiB each)
+    ufomi_chirp chirps[kChirps];  // the last used Bluestein tables
+    float2 *chirp_mem;       // [kChirps][kChirpElems] (6 MiB), allocated with the first
     unsigned long chirp_clock;
     ufomi_block blocks[8];   // at most 512 MiB in all, busy ones included
 };

@@ -91,3 +91,54 @@ def test_one_pipeline_on_two_contexts():
     other = ufo_tasks.Pipeline(_text(W, "backproject"))
     assert torch.equal(other.run(a, x, out_bytes=4 * S * W * W)[0], want)
     del other
+
+
+def _fill(leave):
+    """A buffer that leaves about `leave` bytes of the device free."""
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    free = torch.cuda.mem_get_info()[0]
+    return torch.empty(max(1, free - leave), dtype=torch.uint8, device="cuda")
+
+
+@pytest.mark.parametrize("own", [True, False], ids=["same context", "another context"])
+def test_idle_memory_is_given_back(own):
+    """What a context keeps idle (1 GiB of rows after a stack, a pipeline's blocks) makes room for an allocation
+    that does not fit beside it: a U-Net's, a transform's scratch memory, the next stack's rows."""
+    GiB = 1 << 30
+    st = torch.cuda.current_stream()
+    ctx = ufomi.Context(0, st)
+    user = ctx if own else ufomi.Context(0, st)
+    S, P, W, r = 64, 1800, 2048, 448
+    x = torch.randn(S, P, W, device="cuda")
+    out = torch.empty(S, r, r, device="cuda")
+    roi = dict(n_slices=S, roi_x=800, roi_y=800, roi_width=r, roi_height=r)
+    ctx.bp_parallel(x, W, P, out, **roi)
+    want = out.clone()
+    n = 512
+    img = torch.rand(1, n, n, device="cuda")
+    small = ufomi.Unet(user, 1, n, n, seed=1)
+    ref = torch.empty_like(img)
+    small.forward(img, ref)
+    small.close()
+    # a U-Net of about free + 0.4 GiB: 610 bytes a pixel (float32 output, bf16 images and activations)
+    fill = _fill(2 * GiB)
+    batch = (torch.cuda.mem_get_info()[0] + int(0.4 * GiB)) // (610 * n * n) + 1
+    net = ufomi.Unet(user, batch, n, n, seed=1)
+    got = torch.empty_like(img)
+    net.forward(img, got, batch=1)
+    assert torch.equal(got, ref)
+    net.close()
+    ctx.bp_parallel(x, W, P, out, **roi)   # takes its rows again
+    torch.cuda.synchronize()
+    assert torch.equal(out, want)
+    # two intermediates of a 3-D transform: 1.5 GiB, with less than 1 GiB free
+    del fill
+    z = torch.randn(96, 1024, 1024, device="cuda")
+    spec = torch.empty(96, 1024, 1024, 2, device="cuda")
+    fill = _fill(int(0.8 * GiB))
+    user.fft_nd(z, (1024, 1024, 96), 3, (1024, 1024, 96), spec)
+    torch.cuda.synchronize()
+    assert bool(torch.isfinite(spec[::31, ::101]).all())
+    del fill
+    torch.cuda.empty_cache()

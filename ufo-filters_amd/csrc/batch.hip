@@ -117,7 +117,7 @@ int set_items(ufomi_fbp_batch *b, int tile, int achunk)
     if (items.size() > b->items_cap) {
         if (b->d_items) UFOMI_HIP(hipFree(b->d_items));
         b->d_items = nullptr;
-        UFOMI_HIP(hipMalloc(&b->d_items, items.size() * sizeof(int2)));
+        UFOMI_HIP(ufomi_malloc(b->ctx, (void **) &b->d_items, items.size() * sizeof(int2)));
         b->items_cap = items.size();
     }
     UFOMI_HIP(hipMemcpy(b->d_items, items.data(), items.size() * sizeof(int2), hipMemcpyHostToDevice));
@@ -176,9 +176,9 @@ int check_batch(ufomi_ctx *ctx, ufomi_fbp_batch *b)
 }
 
 template <typename T>
-int upload(T **dst, const T *src, size_t n)
+int upload(ufomi_ctx *ctx, T **dst, const T *src, size_t n)
 {
-    UFOMI_HIP(hipMalloc(dst, n * sizeof(T)));
+    UFOMI_HIP(ufomi_malloc(ctx, (void **) dst, n * sizeof(T)));
     UFOMI_HIP(hipMemcpy(*dst, src, n * sizeof(T), hipMemcpyHostToDevice));
     return UFOMI_OK;
 }
@@ -331,7 +331,7 @@ extern "C" int ufomi_fbp_batch_create(ufomi_ctx *ctx, const ufomi_fbp_request *r
         g.nseg = (int) segs.size();
         b->groups.push_back(g);
         Group &gg = b->groups.back();
-        if ((rc = upload(&gg.d_coef, coef.data(), coef.size())) || (rc = upload(&gg.d_segs, segs.data(), segs.size()))) {
+        if ((rc = upload(ctx, &gg.d_coef, coef.data(), coef.size())) || (rc = upload(ctx, &gg.d_segs, segs.data(), segs.size()))) {
             free_batch(b);
             return rc;
         }
@@ -344,8 +344,8 @@ extern "C" int ufomi_fbp_batch_create(ufomi_ctx *ctx, const ufomi_fbp_request *r
     b->signature = std::string(prop.gcnArchName) + ":" + std::to_string(prop.multiProcessorCount) + ":" +
                    std::to_string(n) + ":" + std::to_string(sig);
     const int zero = 0;
-    if ((rc = upload(&b->d_trig, trig.data(), trig.size())) ||
-        (rc = upload(&b->d_reqs, b->reqs.data(), b->reqs.size())) || (rc = upload(&b->d_counter, &zero, 1)) ||
+    if ((rc = upload(ctx, &b->d_trig, trig.data(), trig.size())) ||
+        (rc = upload(ctx, &b->d_reqs, b->reqs.data(), b->reqs.size())) || (rc = upload(ctx, &b->d_counter, &zero, 1)) ||
         (rc = set_items(b, 32, 16)) || (rc = build_graph(b))) {
         free_batch(b);
         return rc;

@@ -44,6 +44,7 @@ constexpr unsigned kSmallShare = 64;
 constexpr unsigned kLeftOut = 0x7f800000u;  // from here on, a slice's word of maxbits leaves its unit out
 constexpr int kGridY = 65535;  // a grid's second axis: the angles of split_kernel, the slices of absmax_kernel
 // Row workspace of a call: as many groups as fit, one at least; a larger group takes the other path.
+// Partial volumes (fewer than 2048 workgroups' of 256 KiB) come on top.
 constexpr size_t kWorkspace = (size_t) 1 << 30, kGroupMax = (size_t) 4 << 30;
 
 typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
@@ -491,32 +492,6 @@ size_t group_bytes(int W, int P, int planes)
     return (size_t) ((P + 3) / 4 * 4) * planes * (W + 2 * kPad) * kRow;
 }
 
-// The row workspace is shared by all calls of a context: a call waits for the last one's event,
-// whatever stream that was on (on the same one the wait is free, and a new stream may have the
-// handle of one that was destroyed with work pending).
-int acquire_workspace(ufomi_ctx *ctx, size_t bytes)
-{
-    if (!ctx->ws_event)
-        UFOMI_HIP(hipEventCreateWithFlags(&ctx->ws_event, hipEventDisableTiming));
-    if (bytes > ctx->ws_bytes) {
-        if (ctx->ws) {
-            UFOMI_HIP(hipEventSynchronize(ctx->ws_event));
-            UFOMI_HIP(hipFree(ctx->ws));
-            ctx->ws = nullptr;
-            ctx->ws_bytes = 0;
-        }
-        if (ufomi_malloc(ctx, &ctx->ws, bytes) != hipSuccess) {
-            (void) hipGetLastError();  // the caller has a path without it
-            ctx->ws = nullptr;
-            return UFOMI_ERR_MEMORY;
-        }
-        ctx->ws_bytes = bytes;
-    } else {
-        UFOMI_HIP(hipStreamWaitEvent(ctx->stream, ctx->ws_event, 0));
-    }
-    return UFOMI_OK;
-}
-
 // How n slices go over the kernels: n64 units of 64 slices, then n32 of 32, then n16 of 16.
 // Measured at 2048^2 pixels, 720 angles (TGUPS of full units): 64 slices 25.5, 32 slices 22.9,
 // 16 slices 18.2 in f32 storage (16-bit: 37.8, 31.3, 22.4); the interpolating kernel's 8-slice
@@ -569,11 +544,12 @@ template <typename T, int PL> int run(ufomi_ctx *ctx, const T *sino, const ufomi
     const size_t rows_bytes = gb * per_chunk;
     const size_t part_bytes =
         n_split > 1 ? (size_t) n_split * std::min(per_chunk * kSub, n_slices) * plane * sizeof(float) : 0;
-    int rc = acquire_workspace(ctx, head + rows_bytes + part_bytes);
-    if (rc == UFOMI_ERR_MEMORY) return UFOMI_OK;  // *done = 0
+    char *ws = nullptr;
+    int rc = ufomi_workspace(ctx, head + rows_bytes + part_bytes, (void **) &ws);
+    if (rc == UFOMI_ERR_MEMORY) return UFOMI_OK;  // *done = 0: the caller has a path without it
     if (rc) return rc;
-    unsigned *maxbits = (unsigned *) ctx->ws, *nonzero = maxbits + words, *small = nonzero + words;
-    char *rows = (char *) ctx->ws + head;
+    unsigned *maxbits = (unsigned *) ws, *nonzero = maxbits + words, *small = nonzero + words;
+    char *rows = ws + head;
     float *part = n_split > 1 ? (float *) (rows + rows_bytes) : nullptr;
     const int Wp = st.W + 2 * kPad;
     const long elems = (long) st.P * st.W;
@@ -621,7 +597,8 @@ template <typename T, int PL> int run(ufomi_ctx *ctx, const T *sino, const ufomi
     };
     for (int g0 = 0; g0 < groups_all && !rc; g0 += per_chunk) rc = chunk(g0);
     // also where a launch failed: those before it use the workspace
-    UFOMI_HIP(hipEventRecord(ctx->ws_event, ctx->stream));
+    const int end = ufomi_workspace_done(ctx);
+    if (!rc) rc = end;
     if (!rc) *done = n_slices;
     return rc;
 }

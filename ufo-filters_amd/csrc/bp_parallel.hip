@@ -591,7 +591,7 @@ int ufomi_bp_trig(ufomi_ctx *ctx, double angle_offset, double step, unsigned off
             UFOMI_HIP(hipFree(ctx->lut));
             ctx->lut = nullptr;
         }
-        UFOMI_HIP(hipMalloc(&ctx->lut, (size_t) P * sizeof(float2)));
+        UFOMI_HIP(ufomi_malloc(ctx, (void **) &ctx->lut, (size_t) P * sizeof(float2)));
         UFOMI_HIP(hipMemcpy(ctx->lut, h.data(), (size_t) P * sizeof(float2), hipMemcpyHostToDevice));
         ctx->lut_n = P;
         ctx->lut_offset = angle_offset;

@@ -2,6 +2,7 @@
 #include "ufomi_internal.h"
 #include "fft16.h"
 
+#include <algorithm>
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
@@ -40,17 +41,24 @@ int ufomi_enter(ufomi_ctx *ctx)
     return UFOMI_OK;
 }
 
-// Guards the blocks of every context (taken for a list's update only).
-static std::mutex blocks_lock;
+// Every context, and the memory that each keeps idle: its blocks and its row workspace (the lock is
+// taken for a list's update only, and to give idle memory back).
+static std::mutex pool_lock;
+static std::vector<ufomi_ctx *> &contexts = *new std::vector<ufomi_ctx *>;  // outlives every context
 
-static void trim_blocks(ufomi_ctx *ctx)
+static void trim(ufomi_ctx *ctx)
 {
-    std::lock_guard<std::mutex> guard(blocks_lock);
     for (ufomi_block &b : ctx->blocks)
         if (b.ptr && !b.busy) {
             (void) hipFree(b.ptr);
             b = {};
         }
+    if (ctx->ws && !ctx->ws_busy) {
+        (void) hipEventSynchronize(ctx->ws_event);  // its last use may be on any stream
+        (void) hipFree(ctx->ws);
+        ctx->ws = nullptr;
+        ctx->ws_bytes = 0;
+    }
 }
 
 hipError_t ufomi_malloc(ufomi_ctx *ctx, void **ptr, size_t bytes)
@@ -58,10 +66,60 @@ hipError_t ufomi_malloc(ufomi_ctx *ctx, void **ptr, size_t bytes)
     hipError_t e = hipMalloc(ptr, bytes);
     if (e == hipErrorOutOfMemory) {
         (void) hipGetLastError();
-        trim_blocks(ctx);
+        {
+            std::lock_guard<std::mutex> guard(pool_lock);
+            for (ufomi_ctx *c : contexts)
+                if (c->device == ctx->device) trim(c);
+        }
         e = hipMalloc(ptr, bytes);
     }
     return e;
+}
+
+// The row workspace serves one call of the context after the other: each waits for the last one's
+// event, whatever stream that was on (on the same one the wait is free, and a new stream may have
+// the handle of one that was destroyed with work pending).
+int ufomi_workspace(ufomi_ctx *ctx, size_t bytes, void **ptr)
+{
+    if (!ctx->ws_event)
+        UFOMI_HIP(hipEventCreateWithFlags(&ctx->ws_event, hipEventDisableTiming));
+    {
+        std::lock_guard<std::mutex> guard(pool_lock);
+        ctx->ws_busy = 1;
+    }
+    hipError_t e = hipSuccess;
+    if (bytes > ctx->ws_bytes) {
+        if (ctx->ws) {
+            (void) hipEventSynchronize(ctx->ws_event);
+            (void) hipFree(ctx->ws);
+            ctx->ws = nullptr;
+            ctx->ws_bytes = 0;
+        }
+        e = ufomi_malloc(ctx, &ctx->ws, bytes);
+        if (e == hipSuccess) ctx->ws_bytes = bytes;
+        else ctx->ws = nullptr;
+    } else {
+        e = hipStreamWaitEvent(ctx->stream, ctx->ws_event, 0);
+    }
+    if (e != hipSuccess) {
+        (void) hipGetLastError();
+        std::lock_guard<std::mutex> guard(pool_lock);
+        ctx->ws_busy = 0;
+        return ufomi_fail(e == hipErrorOutOfMemory ? UFOMI_ERR_MEMORY : UFOMI_ERR_HIP, "row workspace of %zu bytes: %s",
+                          bytes, hipGetErrorString(e));
+    }
+    *ptr = ctx->ws;
+    return UFOMI_OK;
+}
+
+int ufomi_workspace_done(ufomi_ctx *ctx)
+{
+    hipError_t e = hipEventRecord(ctx->ws_event, ctx->stream);
+    if (e != hipSuccess) (void) hipStreamSynchronize(ctx->stream);  // idle all the same
+    std::lock_guard<std::mutex> guard(pool_lock);
+    ctx->ws_busy = 0;
+    UFOMI_HIP(e);
+    return UFOMI_OK;
 }
 
 int ufomi_scratch(ufomi_ctx *ctx, size_t bytes, void **ptr)
@@ -148,7 +206,8 @@ extern "C" int ufomi_create(int device, ufomi_ctx **out)
         for (int Ns = 16; Ns < N / r0; Ns *= 16) emit(16, Ns);
         emit(r0, N / r0);
     }
-    if (hipMalloc(&ctx->flags, 256) != hipSuccess || hipMalloc(&ctx->twiddles, tw.size() * sizeof(float2)) != hipSuccess ||
+    if (ufomi_malloc(ctx, (void **) &ctx->flags, 256) != hipSuccess ||
+        ufomi_malloc(ctx, (void **) &ctx->twiddles, tw.size() * sizeof(float2)) != hipSuccess ||
         hipMemcpy(ctx->twiddles, tw.data(), tw.size() * sizeof(float2), hipMemcpyHostToDevice) != hipSuccess) {
         free(ctx);
         return ufomi_fail(UFOMI_ERR_HIP, "twiddle table upload failed");
@@ -159,6 +218,10 @@ extern "C" int ufomi_create(int device, ufomi_ctx **out)
         (void) hipFree(ctx->twiddles);
         free(ctx);
         return rc;
+    }
+    {
+        std::lock_guard<std::mutex> guard(pool_lock);
+        contexts.push_back(ctx);
     }
     *out = ctx;
     return UFOMI_OK;
@@ -180,15 +243,15 @@ extern "C" int ufomi_destroy(ufomi_ctx *ctx)
         (void) hipFree(ctx->lut);
     if (ctx->bp_part)
         (void) hipFree(ctx->bp_part);
-    if (ctx->ws) {
-        (void) hipEventSynchronize(ctx->ws_event);  // its last use may be on an earlier stream
-        (void) hipFree(ctx->ws);
+    {
+        std::lock_guard<std::mutex> guard(pool_lock);
+        contexts.erase(std::remove(contexts.begin(), contexts.end(), ctx), contexts.end());
+        trim(ctx);
     }
     if (ctx->ws_event)
         (void) hipEventDestroy(ctx->ws_event);
     if (ctx->chirp_mem)
         (void) hipFree(ctx->chirp_mem);
-    trim_blocks(ctx);
     if (ctx->scratch)
         (void) hipFree(ctx->scratch);
     if (ctx->hscratch)
@@ -250,7 +313,7 @@ extern "C" int ufomi_block_alloc(ufomi_ctx *ctx, size_t bytes, void **out)
     int rc = ufomi_enter(ctx);
     if (rc) return rc;
     {
-        std::lock_guard<std::mutex> guard(blocks_lock);
+        std::lock_guard<std::mutex> guard(pool_lock);
         ufomi_block *best = nullptr;
         size_t held = bytes;
         int empty = 0;
@@ -276,7 +339,7 @@ extern "C" int ufomi_block_alloc(ufomi_ctx *ctx, size_t bytes, void **out)
     }
     if ((rc = ufomi_device_alloc(ctx, bytes, out)))
         return rc;
-    std::lock_guard<std::mutex> guard(blocks_lock);
+    std::lock_guard<std::mutex> guard(pool_lock);
     ufomi_block *empty = nullptr;
     size_t held = bytes;
     for (ufomi_block &b : ctx->blocks) {
@@ -293,7 +356,7 @@ extern "C" int ufomi_block_free(ufomi_ctx *ctx, void *ptr)
     if (rc || !ptr) return rc;
     UFOMI_HIP(hipStreamSynchronize(ctx->stream));
     {
-        std::lock_guard<std::mutex> guard(blocks_lock);
+        std::lock_guard<std::mutex> guard(pool_lock);
         for (ufomi_block &b : ctx->blocks)
             if (b.ptr == ptr) {
                 b.busy = 0;

@@ -49,10 +49,11 @@ struct ufomi_ctx {
     // partial sums of angle-split backprojections of few tiles (grow-only)
     float *bp_part;
     size_t bp_part_bytes;
-    // row workspace of stack backprojections (bp_mfma.hip, grow-only) and the event of its last use
+    // row workspace of stack backprojections (ufomi_workspace) and the event of its last use
     void *ws;
     size_t ws_bytes;
     hipEvent_t ws_event;
+    int ws_busy;             // a call is between ufomi_workspace and ufomi_workspace_done
     ufomi_chirp chirps[kChirps];  // the last used Bluestein tables
     float2 *chirp_mem;       // [kChirps][kChirpElems] (6 MiB), allocated with the first
     unsigned long chirp_clock;
@@ -75,8 +76,13 @@ int ufomi_fail(int code, const char *fmt, ...);
 
 #define UFOMI_CHECK_LAUNCH() UFOMI_HIP(hipGetLastError())
 
-// hipMalloc; when memory is short the context's idle blocks are given back first.
+// hipMalloc; when memory is short, what the contexts of the device keep idle (blocks of pipelines, row
+// workspaces) is given back first.
 hipError_t ufomi_malloc(ufomi_ctx *ctx, void **ptr, size_t bytes);
+// The context's grow-only row workspace, for launches on its stream up to ufomi_workspace_done (which
+// is called whether they succeed or not).  UFOMI_ERR_MEMORY when it cannot be had.
+int ufomi_workspace(ufomi_ctx *ctx, size_t bytes, void **ptr);
+int ufomi_workspace_done(ufomi_ctx *ctx);
 // Device scratch owned by the context (grow-only).
 int ufomi_scratch(ufomi_ctx *ctx, size_t bytes, void **ptr);
 int ufomi_host_scratch(ufomi_ctx *ctx, size_t bytes, void **ptr);

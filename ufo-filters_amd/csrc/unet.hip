@@ -491,7 +491,7 @@ namespace {
 
 int dalloc(ufomi_unet *n, size_t bytes, void **p)
 {
-    hipError_t e = hipMalloc(p, bytes ? bytes : 1);
+    hipError_t e = ufomi_malloc(n->ctx, p, bytes ? bytes : 1);
     if (e != hipSuccess)
         return ufomi_fail(UFOMI_ERR_MEMORY, "cannot allocate %zu bytes for the U-Net: %s", bytes,
                           hipGetErrorString(e));

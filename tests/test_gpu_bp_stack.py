@@ -92,6 +92,30 @@ def test_geometry_and_pitches(ctx, torch_dev, props):
     np.testing.assert_array_equal(flat[0][:, :rw * rh].reshape(S, rh, rw), got.cpu().numpy())
 
 
+@pytest.mark.parametrize("S,P,W,roi,storage,matrix", [
+    (16, 800, 2048, 320, "f32", False), (16, 800, 2048, 1024, "f32", True),
+    (24, 900, 2048, 384, "f16", False), (24, 900, 2048, 768, "f16", True),
+    (64, 720, 4096, 256, "bf16", False), (64, 720, 4096, 512, "bf16", True),
+])
+def test_small_regions_of_wide_detectors(ctx, torch_dev, S, P, W, roi, storage, matrix):
+    """Regions too small to pay for laying out whole rows stay with the interpolating kernel (f16: the one with
+    half staging, as before)."""
+    import torch
+    x = _stack(torch_dev, S, P, W, storage, seed=14)
+    props = dict(roi_x=(W - roi) // 2, roi_y=(W - roi) // 3, roi_width=roi, roi_height=roi)
+    got, ref = _both(ctx, torch_dev, x, storage, **props)
+    if storage == "f16" and not matrix:
+        try:
+            ctx.bp_configure(8, 8, 0)
+            ctx.bp_parallel(x, W, P, ref, n_slices=S, dtype=ufomi.F16, **props)
+        finally:
+            ctx.bp_configure(0, 0, 0)
+    assert torch.equal(got, ref) != matrix
+    # float32 coordinates of the interpolating kernel: 2^-14 pixels at 1024 to 2048, the samples' difference is
+    # 1.4 of their size and one of two roundings counts
+    assert rel_l2(got.cpu().numpy(), ref.cpu().numpy()) < 2.0 ** -14
+
+
 @pytest.mark.parametrize("S,P,W,roi,matrix", [
     (12, 65532, 16, 36, True),     # the largest angle count, rounded up to fours, of the layout's grid
     (12, 65533, 16, 36, False),

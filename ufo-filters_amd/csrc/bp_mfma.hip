@@ -518,10 +518,30 @@ Units units_of(int n)
     return u;
 }
 
+// Whether the units are faster than the interpolating kernel for them.  The layout reads and writes
+// whole rows whatever the region of interest needs of them, so a small region of a wide detector
+// does not pay for it.  Rates of updates (per us, in 1e6) as above, of the interpolating kernel as
+// it reaches them on regions of 256 to 1024 pixels, and microseconds per 1e6 samples of the layout
+// (a slice read, a slice of a group of 32 written).  Measured over 12 to 64 slices of 400 to 3000
+// angles x 512 to 4096 pixels, regions of 128 to 1024: one of 78 cases goes the slower way, by 3%.
+// In us, matrix cores / interpolating kernel, 64 slices of 1800 x 2048 in f32: 724 / 240 for 128^2
+// pixels, 922 / 779 for 256^2, 1454 / 1748 for 384^2; 16 slices 479 / 451 for 384^2, 644 / 776 for 512^2.
+bool pays(const ufomi_bp_stack &st, const Units &u)
+{
+    const bool f32 = st.dtype == UFOMI_F32;
+    const double interp = st.dtype == UFOMI_F16 ? 14.5 : 10.8;
+    const double r64 = f32 ? 25.5 : 37.8, r32 = f32 ? 22.9 : 31.3, r16 = f32 ? 18.2 : 22.4;
+    const double read = f32 ? 1.77 : 1.0, write = f32 ? 0.64 : 1.1;
+    const double updates = 1e-6 * ((st.roi_w + kTile - 1) / kTile) * ((st.roi_h + kTile - 1) / kTile) * kTile * kTile * st.P;
+    const double layout = 1e-6 * st.P * st.W * (read * u.slices + write * ((u.slices + kSub - 1) / kSub * kSub));
+    return updates * (u.n64 * 64 / r64 + u.n32 * 32 / r32 + u.n16 * 16 / r16) + layout <
+           updates * ((u.slices + 7) / 8 * 8) / interp;
+}
+
 template <typename T, int PL> int run(ufomi_ctx *ctx, const T *sino, const ufomi_bp_stack &st, int *done)
 {
     const Units all = units_of(st.n_slices);
-    if (!all.slices) return UFOMI_OK;
+    if (!all.slices || !pays(st, all)) return UFOMI_OK;
     const int n_slices = all.slices;
     const size_t gb = group_bytes(st.W, st.P, PL);
     const int groups_all = (n_slices + kSub - 1) / kSub;

@@ -721,7 +721,8 @@ int bp_parallel_impl(ufomi_ctx *ctx, const void *d_sino, int dtype, int W, int P
     // us, this kernel / the matrix cores, f32 storage: 24 slices of 400^2 x 180 (6.9e8 updates)
     // 100 / 102, 12 of 400^2 x 500 (9.6e8) 162 / 132, 64 of 1024^2 x 800 (5.4e10) 4824 / 2336; f16
     // storage, whose half staging is faster here: 24 of 400^2 x 500 (1.9e9) 167 / 172, 32 (2.6e9)
-    // 240 / 185, 64 of 1024^2 x 800 3486 / 1625.
+    // 240 / 185, 64 of 1024^2 x 800 3486 / 1625.  These are whole slices; small regions of a wide
+    // detector may stay here above the line too (pays() there).
     const double updates = (double) n_slices * roi_w * roi_h * P_in;
     if (!fixed && !ctx->bp_slices && !ctx->bp_chunk && n_slices >= 12 &&
         updates >= (dtype == UFOMI_F16 ? 2.5e9 : 1e9)) {

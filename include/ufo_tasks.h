@@ -127,7 +127,10 @@ size_t ufomi_requisition_elements(const UfomiRequisition *req);
  * items of a backproject stage run as one multi-slice launch.  General
  * backprojection consumes all items (projections) and emits its slices.
  * The output items are written contiguously to d_out (at most out_capacity
- * bytes); *n_out and *out_req describe them.
+ * bytes); *n_out and *out_req describe them.  The last stage may write d_out
+ * itself: a run that fails there for want of memory or by a device error can
+ * leave it partly written.  Every other failure (arguments, sizes, an earlier
+ * stage) leaves it untouched.
  *
  * A first stage `read` produces the input items from files (d_in, in_req and
  * n_items are then ignored and may be NULL / 0); a last stage `write` writes

@@ -58,6 +58,18 @@ def test_destinations_agree(last):
     assert rc == 0 and torch.equal(both[:n], want)
 
 
+@pytest.mark.parametrize("tail", [" ! backproject num-projections=5", " ! backproject ! ifft dimensions=1"])
+def test_failures_leave_the_output(tail):
+    """Arguments and sizes are checked before the stage that writes the caller's memory starts."""
+    W, P, S = 65, 9, 5
+    ctx = ufomi.Context(0, torch.cuda.current_stream())
+    x = torch.randn(S, P, W, device="cuda")
+    out = torch.full((4 * S * W * W,), 7.0, device="cuda")
+    rc, _ = _run(ctx, _text(W, "ifft") + tail, x, out.data_ptr(), 4 * out.numel())
+    torch.cuda.synchronize()
+    assert rc != 0 and bool((out == 7.0).all())
+
+
 def test_blocks_over_sizes_and_streams():
     """Batches that grow, shrink and exceed what the context keeps, on two streams in turn."""
     a, b = torch.cuda.Stream(), torch.cuda.Stream()

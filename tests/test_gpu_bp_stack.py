@@ -55,6 +55,7 @@ def test_units_vs_oracle(ctx, torch_dev, S, P, W, storage):
     got, ref = _both(ctx, torch_dev, x, storage, axis_pos=W / 2.0 + 0.25)
     got, ref = got.cpu().numpy(), ref.cpu().numpy()
     assert np.isfinite(got).all()
+    assert not np.array_equal(got, ref)  # the matrix cores ran: they sum in another order
     for s in range(S):
         assert rel_l2(got[s], ref[s]) < 1e-5, s
     s = S // 2
@@ -66,18 +67,21 @@ def test_units_vs_oracle(ctx, torch_dev, S, P, W, storage):
 
 @pytest.mark.parametrize("props", [
     dict(axis_pos=150.25, roi_x=33, roi_y=7, roi_width=301, roi_height=215, angle_offset=0.7),
-    dict(angle_step=0.013, offset=11, num_projections=700),
+    dict(angle_step=0.013, offset=11, num_projections=900),
     dict(axis_pos=1.5, roi_width=420, roi_height=300),   # most of the image off the detector
 ])
 def test_geometry_and_pitches(ctx, torch_dev, props):
     import torch
-    S, P, W = 24, 600, 300
+    S, P, W = 24, 800, 300  # at least 1.2e9 updates
     x = _stack(torch_dev, S, P, W, seed=5)
     rw, rh = props.get("roi_width") or W, props.get("roi_height") or W
     wide = torch.zeros((S, P * W + 37), device=torch_dev)
     wide[:, :P * W] = x.view(S, -1)
     pitch = rw * rh + 3  # slices of the output off the 16-byte alignment
-    got, _ = _both(ctx, torch_dev, x, "f32", **props)
+    got, ref = _both(ctx, torch_dev, x, "f32", **props)
+    assert not torch.equal(got, ref)  # the matrix cores ran: they sum in another order
+    exact = oracle.bp_texture_f64(x[7].cpu().numpy(), **props)
+    assert rel_l2(got[7].cpu().numpy(), exact) < 1e-5
     flat = []
     for config in ((0, 0, 0), (8, 8, -1)):
         try:
@@ -137,6 +141,25 @@ def test_launch_limits(ctx, torch_dev, S, P, W, roi, matrix):
     if not matrix or S < 100:
         exact = oracle.bp_texture_f64(x[S // 2].cpu().numpy(), axis_pos=W / 2.0, roi_width=roi, roi_height=roi)
         assert rel_l2(got[S // 2].cpu().numpy(), exact) < 1e-5 + 2.0 ** -24 * P ** 0.5
+
+
+def test_chunks_of_the_workspace(ctx, torch_dev):
+    """Rows above 1 GiB go in chunks: two of 64 slices here, and one of 41 as units of 32 and 16 (padded).  An
+    Inf leaves out the second chunk's unit and a large sample the third one's first: the interpolating kernel's
+    bits are there, and nowhere else."""
+    import torch
+    S, P, W, roi = 169, 3000, 1300, 260
+    x = torch.randn((S, P, W), device=torch_dev, generator=torch.Generator(device=torch_dev).manual_seed(15))
+    x[70, 5, 600] = float("inf")
+    x[150, 7, 650] = 1e20
+    got, ref = _both(ctx, torch_dev, x, roi_x=520, roi_y=515, roi_width=roi, roi_height=roi - 3)
+    finite = torch.isfinite(ref)
+    assert bool((torch.isfinite(got) == finite).all())
+    got[~finite] = ref[~finite] = 0.0
+    for s in range(S):
+        # coordinates of 1300 pixels round at up to 2^-14 pixels there, a fifth of that on average
+        assert rel_l2(got[s].cpu().numpy(), ref[s].cpu().numpy()) < 2e-5, s
+        assert torch.equal(got[s], ref[s]) == (64 <= s < 160), s
 
 
 @pytest.mark.parametrize("storage", ["f32", "f16", "bf16"])

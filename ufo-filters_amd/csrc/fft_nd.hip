@@ -50,14 +50,16 @@ struct Pass {
 __device__ __forceinline__ float2 load_as_complex(const float *p, long o) { return make_float2(p[o], 0.0f); }
 __device__ __forceinline__ float2 load_as_complex(const float2 *p, long o) { return p[o]; }
 
+constexpr int kSplitB = 4;  // radix-4 butterflies a thread holds in a split pass of 128 to 1024 points
+
 // A pass of the four-step split: lines through LDS.  Lines along axis 0 are contiguous; of strided
 // lines a block takes G neighbouring ones, so that one row of its tile is G consecutive values.
-template <int BB, int DIR, typename InT, bool OUT_REAL>
+template <int DIR, typename InT, bool OUT_REAL>
 __global__ __launch_bounds__(kThreads) void axis_dft_kernel(const InT *__restrict__ in, void *__restrict__ out_, Pass g,
                                                             const float2 *__restrict__ tw)
 {
     extern __shared__ float2 lds[];
-    const int TF = g.L / (4 * BB);
+    const int TF = g.L / (4 * kSplitB);
     const int f = threadIdx.x / TF, t = threadIdx.x - f * TF;
     const int ablocks = (g.A + g.G - 1) / g.G;
     const int b = blockIdx.x / ablocks;
@@ -82,7 +84,7 @@ __global__ __launch_bounds__(kThreads) void axis_dft_kernel(const InT *__restric
         lds[gl * g.Ls + i] = v;
     }
     __syncthreads();
-    lds_fft<BB, DIR>(lds + f * g.Ls, g.L, g.log2L, t, TF, tw);
+    lds_fft<kSplitB, DIR>(lds + f * g.Ls, g.L, g.log2L, t, TF, tw);
 
     const int total_out = g.G * g.n_out;
     for (int idx = threadIdx.x; idx < total_out; idx += kThreads) {
@@ -256,7 +258,6 @@ void bluestein_tables(int M, int L, int dir, float2 *chirp, float2 *kern)
 
 struct PassSpec {
     Pass g;
-    int BB;              // four-step split only
     bool chirp;
     int M;
     const float2 *tables;  // chirp[M], then the kernel spectrum
@@ -312,24 +313,12 @@ int make_pass(int axis, const int S[3], const int D[3], const int E[3], int n_in
 }
 
 template <int DIR, typename InT, bool OUT_REAL>
-int launch_bb(hipStream_t s, const PassSpec &ps, const void *in, void *out, const float2 *tw)
+int launch_split(hipStream_t s, const Pass &g, const void *in, void *out, const float2 *tw)
 {
-    const Pass &g = ps.g;
     const unsigned blocks = (unsigned) ((long) g.Bn * ((g.A + g.G - 1) / g.G));
     const size_t lds = (size_t) g.G * g.Ls * sizeof(float2);
-    switch (ps.BB) {
-#define UFOMI_AXIS_CASE(BBV)                                                                                       \
-    case BBV:                                                                                                      \
-        hipLaunchKernelGGL((axis_dft_kernel<BBV, DIR, InT, OUT_REAL>), dim3(blocks), dim3(kThreads), lds, s,       \
-                           (const InT *) in, out, g, tw);                                                          \
-        break;
-        UFOMI_AXIS_CASE(1)
-        UFOMI_AXIS_CASE(2)
-        UFOMI_AXIS_CASE(4)
-        UFOMI_AXIS_CASE(8)
-#undef UFOMI_AXIS_CASE
-    default: return ufomi_fail(UFOMI_ERR_ARG, "internal: no axis kernel for %d butterflies", ps.BB);
-    }
+    hipLaunchKernelGGL((axis_dft_kernel<DIR, InT, OUT_REAL>), dim3(blocks), dim3(kThreads), lds, s, (const InT *) in, out,
+                       g, tw);
     UFOMI_CHECK_LAUNCH();
     return UFOMI_OK;
 }
@@ -446,6 +435,7 @@ int setup_scratch(ufomi_ctx *ctx, PassSpec *ps, int np, int dir, size_t tmp_elem
 //   pass 1: for every n2, an N1-point transform over n1 (stride N2), times
 //           exp(dir 2 pi i n2 k1 / N), into [k1][n2];
 //   pass 2: for every k1, an N2-point transform over n2, written to k1 + N1 k2.
+// N is 2^14 to 2^20, N1 and N2 128 to 1024.
 // Row r of the input holds `valid` elements at pitch `in_pitch`; row r of the
 // output holds the first `keep` outputs at pitch `out_pitch`.
 constexpr long kMaxSplit = 1L << 20;
@@ -454,12 +444,12 @@ void split_pass(Pass &g, int L)
 {
     g.L = L;
     g.log2L = ufomi_log2(L);
+    g.G = 1024 * kSplitB / L;
+    g.Ls = L + 1;
     g.scale = 1.0f;
     g.flat_in = g.flat_out = 0;
     g.tw_n = 0;
 }
-
-int bb_of(int L) { return L >= 8192 ? 8 : std::min(4, L / 16); }
 
 template <int DIR, typename InT, bool OUT_REAL>
 int split_passes(ufomi_ctx *ctx, const void *in, long in_pitch, long valid, int rows, int N, long keep,
@@ -469,12 +459,8 @@ int split_passes(ufomi_ctx *ctx, const void *in, long in_pitch, long valid, int 
     const int N1 = 1 << (lg / 2), N2 = N / N1;
     if (rows <= 0)
         return ufomi_fail(UFOMI_ERR_ARG, "invalid transform rows");
-    PassSpec p1{}, p2{};
-    Pass &a = p1.g, &b = p2.g;
+    Pass a{}, b{};
     split_pass(a, N1);
-    p1.BB = bb_of(N1);
-    a.G = 1024 * p1.BB / N1;
-    a.Ls = a.G > 1 ? N1 + 1 : N1;
     a.A = N2, a.Bn = rows;
     a.in_a = 1, a.in_e = N2, a.in_b = in_pitch;
     a.n_in = N1, a.flat_in = valid;
@@ -482,9 +468,6 @@ int split_passes(ufomi_ctx *ctx, const void *in, long in_pitch, long valid, int 
     a.n_out = N1;
     a.tw_n = N;
     split_pass(b, N2);
-    p2.BB = bb_of(N2);
-    b.G = 1024 * p2.BB / N2;
-    b.Ls = b.G > 1 ? N2 + 1 : N2;
     b.A = N1, b.Bn = rows;
     b.in_a = N2, b.in_e = 1, b.in_b = N;
     b.n_in = N2;
@@ -496,9 +479,9 @@ int split_passes(ufomi_ctx *ctx, const void *in, long in_pitch, long valid, int 
         if (blocks <= 0 || blocks >= (1L << 31))
             return ufomi_fail(UFOMI_ERR_ARG, "transform of %d rows does not fit one launch", rows);
     }
-    int rc = launch_bb<DIR, InT, false>(ctx->stream, p1, in, tmp, ctx->twiddles);
+    int rc = launch_split<DIR, InT, false>(ctx->stream, a, in, tmp, ctx->twiddles);
     if (rc) return rc;
-    return launch_bb<DIR, float2, OUT_REAL>(ctx->stream, p2, tmp, out, ctx->twiddles);
+    return launch_split<DIR, float2, OUT_REAL>(ctx->stream, b, tmp, out, ctx->twiddles);
 }
 
 template <int DIR, typename InT, bool OUT_REAL>

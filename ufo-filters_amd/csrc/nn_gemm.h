@@ -777,7 +777,7 @@ static __device__ __align__(16) unsigned char g_conv_zero16[16];
 // past cout load g_conv_zero16), and so do the chunk's BN x 9 x 32 weights, so
 // the tap loop issues no global loads: 78 KB of LDS for 64 channels x 64 pixels
 // (two workgroups per CU, as the registers allow), 40 KB for 32 channels x 32
-// pixels (four).  Other shapes take the weight fragments from L2 a tap ahead.
+// pixels (four).
 // With LDS_OUT the finished tile leaves through LDS in 16-byte vectors, with the
 // optional 2 x 2 max pool (4 pooled rows).  Needs W a multiple of TX, H a
 // multiple of 8, cin a multiple of 32.  The accumulators stay in VGPRs (two
@@ -789,15 +789,14 @@ __global__ __launch_bounds__(512 / RPW) __attribute__((amdgpu_waves_per_eu(4 / R
     constexpr int WAVES = TY / RPW, NTH = 64 * WAVES;
     constexpr int NVEC = PY * PX * 4;        // 16-byte vectors of a patch (32 channels)
     constexpr int PINS = (NVEC + 63) / 64;   // wave loads per patch
-    constexpr bool WL = NT >= 4 || TX <= 32;  // weights staged in LDS
-    constexpr int WV = WL ? BN * 36 : 0;    // 16-byte vectors of a chunk's weights: [BN][9 taps][4]
+    constexpr int WV = BN * 36;             // 16-byte vectors of a chunk's weights: [BN][9 taps][4]
     constexpr int WINS = (WV + 63) / 64;     // wave loads per chunk of weights
     constexpr int STAGED = (PINS + WINS) * 64;
     constexpr int OUTV = TY * TX * BN / 8;   // 16-byte vectors of the finished tile
     constexpr int SH = (!LDS_OUT || STAGED > OUTV) ? STAGED : OUTV;
     __shared__ bf16x8 sh[SH];
     bf16x8 *patch = sh;
-    [[maybe_unused]] bf16x8 *wts = sh + PINS * 64;
+    bf16x8 *wts = sh + PINS * 64;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int r = lane & 15, q = lane >> 4;
     const int W = 1 << op.lw, H = 1 << op.lh;
@@ -835,7 +834,7 @@ __global__ __launch_bounds__(512 / RPW) __attribute__((amdgpu_waves_per_eu(4 / R
     const bf16 *ibase = op.in.ptr + pix0 * op.in.cs + op.in.c0;
     const bf16 *wbase = op.w + n0 * (9L << op.lcin);
     int poff[PJ];
-    [[maybe_unused]] int woff[WJ > 0 ? WJ : 1];
+    int woff[WJ];
 #pragma unroll
     for (int k = 0; k < PJ; k++) {
         const int v = (wave + WAVES * k) * 64 + lane;
@@ -867,28 +866,13 @@ __global__ __launch_bounds__(512 / RPW) __attribute__((amdgpu_waves_per_eu(4 / R
 #pragma unroll
         for (int k = 0; k < WJ; k++) {
             const int j = wave + WAVES * k;
-            if (WL && j < WINS) {
+            if (j < WINS) {
                 const void *src = woff[k] != kNone ? (const void *) (wbase + woff[k] + c0) : zero16;
                 __builtin_amdgcn_global_load_lds(src, (lds_void *) (wts + j * 64), 16, 0, 0);
             }
         }
     };
 
-    // weight fragments from L2 when they are not staged (32 channels on 64-pixel tiles): row
-    // n0 + 16 j + r, loaded a tap ahead
-    const bf16 *wrow[NT];
-    bool wok[NT];
-#pragma unroll
-    for (int j = 0; j < NT; j++) {
-        const long co = n0 + j * 16 + r;
-        wok[j] = co < op.cout;
-        wrow[j] = op.w + (wok[j] ? co : 0) * (9L << op.lcin);
-    }
-    auto load_b = [&](bf16x8 *bfr, int tap, int c0) {
-#pragma unroll
-        for (int j = 0; j < NT; j++)
-            bfr[j] = wok[j] ? ld8(wrow[j] + ((long) tap << op.lcin) + c0 + 8 * q) : zero8();
-    };
     f32x4 acc[MT][NT];
 #pragma unroll
     for (int i = 0; i < MT; i++)
@@ -899,10 +883,8 @@ __global__ __launch_bounds__(512 / RPW) __attribute__((amdgpu_waves_per_eu(4 / R
     for (int ch = 0; ch < nchunks; ch++) {
         const int c0 = ch * 32;
         stage(c0);
-        bf16x8 bcur[NT], bnext[NT];
-        if constexpr (!WL) load_b(bcur, 0, c0);
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __syncthreads();  // patch (and weights) of chunk ch in LDS
+        __syncthreads();  // patch and weights of chunk ch in LDS
         // rows of taps: dy in a loop, dx unrolled (the patch and weight offsets of a row are
         // immediates from one base)
 #pragma unroll 1
@@ -911,14 +893,8 @@ __global__ __launch_bounds__(512 / RPW) __attribute__((amdgpu_waves_per_eu(4 / R
         for (int dx = 0; dx < 3; dx++) {
             const int tap = 3 * dy + dx;  // patch offsets (dy, dx), 0..2
             bf16x8 bfr[NT];
-            if constexpr (WL) {
 #pragma unroll
-                for (int j = 0; j < NT; j++) bfr[j] = wts[(16 * j + r) * 36 + tap * 4 + q];
-            } else {
-                if (tap < 8) load_b(bnext, tap + 1, c0);
-#pragma unroll
-                for (int j = 0; j < NT; j++) bfr[j] = bcur[j];
-            }
+            for (int j = 0; j < NT; j++) bfr[j] = wts[(16 * j + r) * 36 + tap * 4 + q];
             bf16x8 afr[MT];
 #pragma unroll
             for (int i = 0; i < MT; i++)
@@ -929,10 +905,6 @@ __global__ __launch_bounds__(512 / RPW) __attribute__((amdgpu_waves_per_eu(4 / R
 #pragma unroll
                 for (int j = 0; j < NT; j++)
                     acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bfr[j], afr[i], acc[i][j], 0, 0, 0);
-            if constexpr (!WL) {
-#pragma unroll
-                for (int j = 0; j < NT; j++) bcur[j] = bnext[j];
-            }
         }
         __syncthreads();  // every wave done with this chunk before the next is staged
     }

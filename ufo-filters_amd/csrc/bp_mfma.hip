@@ -450,7 +450,9 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NT == 1
     // D of a block: lane holds voxels (0 .. 3, g) of slice l16
     const float fp = (float) p_norm;
     out += (long) blockIdx.y * part_pitch;
-    const bool vec = ((roi_w | out_pitch | part_pitch) & 3) == 0 && ((unsigned long) out & 15) == 0;
+    // 16-byte stores need 4-byte alignment only; written as four, a slice of odd width took 24 slices
+    // of 400 x 701 in f16 storage from 277 to 382 us
+    typedef float vec_t __attribute__((ext_vector_type(4), aligned(4)));
 #pragma unroll
     for (int n = 0; n < NG * NT; n++) {
         const int sl = slice0 + (n / NT) * kSub + (n % NT) * 16 + l16;
@@ -463,8 +465,8 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NT == 1
 #pragma unroll
             for (int k = 0; k < 4; k++) r[k] = (acc[i][n][k] * inv) * 3.14159274101257324219f / fp;
             float *o = out + (long) sl * out_pitch + (long) y * roi_w + x;
-            if (vec && x + 3 < roi_w) {
-                *(float4_t *) o = r;
+            if (x + 3 < roi_w) {
+                *(vec_t *) o = r;
             } else {
 #pragma unroll
                 for (int k = 0; k < 4; k++)

@@ -100,10 +100,11 @@ def test_geometry_and_pitches(ctx, torch_dev, props):
     (16, 800, 2048, 320, "f32", False), (16, 800, 2048, 1024, "f32", True),
     (24, 900, 2048, 384, "f16", False), (24, 900, 2048, 768, "f16", True),
     (64, 720, 4096, 256, "bf16", False), (64, 720, 4096, 512, "bf16", True),
+    (100, 180, 256, 256, "f32", False), (96, 180, 256, 256, "f32", True),  # leftovers' own launch, none
 ])
-def test_small_regions_of_wide_detectors(ctx, torch_dev, S, P, W, roi, storage, matrix):
-    """Regions too small to pay for laying out whole rows stay with the interpolating kernel (f16: the one with
-    half staging, as before)."""
+def test_small_work(ctx, torch_dev, S, P, W, roi, storage, matrix):
+    """Regions too small to pay for laying out whole rows, and stacks too small to pay for a launch of leftover
+    slices, stay with the interpolating kernel (f16: the one with half staging, as before)."""
     import torch
     x = _stack(torch_dev, S, P, W, storage, seed=14)
     props = dict(roi_x=(W - roi) // 2, roi_y=(W - roi) // 3, roi_width=roi, roi_height=roi)

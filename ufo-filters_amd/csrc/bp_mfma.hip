@@ -522,12 +522,15 @@ Units units_of(int n)
 
 // Whether the units are faster than the interpolating kernel for them.  The layout reads and writes
 // whole rows whatever the region of interest needs of them, so a small region of a wide detector
-// does not pay for it.  Rates of updates (per us, in 1e6) as above, of the interpolating kernel as
+// does not pay for it; and up to 8 leftover slices take a launch of their own, too few workgroups
+// to hide its 60 us.  Rates of updates (per us, in 1e6) as above, of the interpolating kernel as
 // it reaches them on regions of 256 to 1024 pixels, and microseconds per 1e6 samples of the layout
-// (a slice read, a slice of a group of 32 written).  Measured over 12 to 64 slices of 400 to 3000
-// angles x 512 to 4096 pixels, regions of 128 to 1024: one of 78 cases goes the slower way, by 3%.
+// (a slice read, a slice of a group of 32 written).  Measured over 12 to 128 slices of 90 to 3000
+// angles x 256 to 4096 pixels, whole and regions of 128 to 1024: 5 of 893 stacks go the slower way
+// by more than 4%, at most 10%.
 // In us, matrix cores / interpolating kernel, 64 slices of 1800 x 2048 in f32: 724 / 240 for 128^2
-// pixels, 922 / 779 for 256^2, 1454 / 1748 for 384^2; 16 slices 479 / 451 for 384^2, 644 / 776 for 512^2.
+// pixels, 922 / 779 for 256^2, 1454 / 1748 for 384^2; 16 slices 479 / 451 for 384^2, 644 / 776 for 512^2;
+// 100 slices (4 leftover) of 180 x 256 192 / 158.
 bool pays(const ufomi_bp_stack &st, const Units &u)
 {
     const bool f32 = st.dtype == UFOMI_F32;
@@ -536,8 +539,9 @@ bool pays(const ufomi_bp_stack &st, const Units &u)
     const double read = f32 ? 1.77 : 1.0, write = f32 ? 0.64 : 1.1;
     const double updates = 1e-6 * ((st.roi_w + kTile - 1) / kTile) * ((st.roi_h + kTile - 1) / kTile) * kTile * kTile * st.P;
     const double layout = 1e-6 * st.P * st.W * (read * u.slices + write * ((u.slices + kSub - 1) / kSub * kSub));
-    return updates * (u.n64 * 64 / r64 + u.n32 * 32 / r32 + u.n16 * 16 / r16) + layout <
-           updates * ((u.slices + 7) / 8 * 8) / interp;
+    const double rest = u.slices < st.n_slices ? 60.0 + 0.6 * updates * 8 / interp : 0.0;
+    return updates * (u.n64 * 64 / r64 + u.n32 * 32 / r32 + u.n16 * 16 / r16) + layout + rest <
+           updates * ((st.n_slices + 7) / 8 * 8) / interp;
 }
 
 template <typename T, int PL> int run(ufomi_ctx *ctx, const T *sino, const ufomi_bp_stack &st, int *done)

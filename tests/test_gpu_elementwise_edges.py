@@ -20,8 +20,11 @@ def _dev(x, torch_dev, shift=0):
 
 
 @pytest.mark.parametrize("n,h,w,shift", [(1, 3, 8, 0), (7, 5, 4, 0), (8, 2, 6, 0), (9, 1, 1028, 0), (17, 3, 5, 0),
-                                         (9, 4, 16, 1), (20, 2, 2, 0)])
-@pytest.mark.parametrize("sino,nd,nf", [(False, 1, 1), (False, 3, 10), (True, 12, 2), (True, 1, 1)])
+                                         (9, 4, 16, 1), (20, 2, 2, 0),
+                                         # runs of 2, 4 and 8 items need 1024 workgroups at least
+                                         (2047, 1, 6, 0), (4095, 1, 4, 0), (8190, 1, 5, 0), (8185, 1, 4, 0)])
+@pytest.mark.parametrize("sino,nd,nf", [(False, 1, 1), (False, 3, 10), (True, 12, 2), (True, 1, 1),
+                                        (False, 4091, 8188)])
 def test_flat_field_runs(ctx, torch_dev, n, h, w, shift, sino, nd, nf):
     rng = np.random.default_rng(n * 100 + w)
     nd, nf = min(nd, n), min(nf, n)
@@ -33,7 +36,8 @@ def test_flat_field_runs(ctx, torch_dev, n, h, w, shift, sino, nd, nf):
     ctx.flat_field_correct(_dev(data, torch_dev, shift), w, h, n, _dev(dark, torch_dev), nd, _dev(flat, torch_dev), nf,
                            out, sinogram_input=sino, absorption_correct=True, dark_scale=0.5, flat_scale=1.5)
     got = out.cpu().numpy()
-    for i in range(n):
+    assert np.isfinite(got).all()
+    for i in range(n) if n < 100 else [*range(20), *range(max(nd - 9, 0), min(nd + 9, n)), *range(n - 20, n)]:
         ref = oracle.flat_field_correct_ref32(data[i:i + 1], dark[min(i, nd - 1)], flat[min(i, nf - 1)], True, False,
                                               False, 0.5, 1.5)[0]
         assert rel_l2(got[i], ref) < 1e-6, i  # one rounding of logf (2 ulp) over the oracle's

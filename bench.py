@@ -220,7 +220,8 @@ def fbp_parallel(args, ctx, torch, np, ufomi, S, W, P, filt_name, noise, storage
     first = storages[0]
 
     def on_mfma(st):
-        # stacks go to the matrix cores, unless a tile configuration is forced
+        # stacks go to the matrix cores, unless a tile configuration is forced (whole slices of this
+        # much work always pay for the layout of their rows)
         return not args.bp_config and S >= 12 and updates >= (2.5e9 if st == "f16" else 1e9)
 
     def kname(st):
@@ -293,7 +294,9 @@ def fbp_parallel(args, ctx, torch, np, ufomi, S, W, P, filt_name, noise, storage
     hbm_bytes = float(S) * P * W * (4 if first == "f32" else 2) + float(S) * W * W * 4
     return dict(updates=updates, wall=r["wall"], bp_ms=r["bp_ms"], kernel=kernel, bytes_per_update=bpu,
                 mfma_flops_per_update=mfma, hbm_bytes=hbm_bytes, extra=extra, cpu=cpu, accuracy=accuracy,
-                workload=workload, dtype="f32" if first == "f32" else "f32 accumulate, %s storage" % first,
+                workload=workload, dtype=("f32" if not on_mfma(first) else "f32 (backprojection: samples and weights as "
+                                          "pairs of f16, 22 bits, f32 sums)")
+                if first == "f32" else "f32 accumulate, %s storage" % first,
                 config={"slices": S, "angles": P, "detector": W, "fft_size": N, "storage": first, "filter": filt_name},
                 traffic_key="%s %dx%dx%d %s" % (kernel, S, P, W, first),
                 metric="GUPS (voxel*proj/s) for FBP")

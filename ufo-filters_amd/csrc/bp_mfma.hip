@@ -213,7 +213,8 @@ __device__ __forceinline__ short4_t read_tr(const LdsChar *p)
 // 16 bytes per lane from src (uniform) + offset to LDS address dst (uniform) + 16 lane, in flight
 // until the caller's vmcnt wait.  Written out because the compiler, which cannot tell the two
 // staging buffers apart, waits for the builtin's loads before the next LDS read (64 slices of
-// 720 x 2048: 8.6 ms with that wait, 7.4 without).  Nothing else here uses m0.
+// 720 x 2048: 8.6 ms with that wait, 7.4 without).  Nothing else here uses m0 (a reserved
+// register, so not to be declared).
 __device__ __forceinline__ void load_lds(unsigned dst, const char *src, unsigned offset)
 {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tglobal_load_lds_dwordx4 %1, %2"

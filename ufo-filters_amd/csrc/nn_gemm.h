@@ -39,7 +39,8 @@ __device__ __forceinline__ bf16x8 zero8()
 __device__ __forceinline__ bf16x8 ld8(const bf16 *p) { return *reinterpret_cast<const bf16x8 *>(p); }
 
 // 16 bytes from each lane's address to LDS address dst (uniform) + 16 lane, in flight until the
-// caller's vmcnt wait; the builtin would wait before the next LDS read.
+// caller's vmcnt wait; the builtin would wait before the next LDS read.  A kernel that uses it does
+// not use the builtin or anything else that sets m0 (a reserved register, so not to be declared).
 __device__ __forceinline__ void load_lds_async(unsigned dst, const void *src)
 {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(dst), "v"(src) : "memory");

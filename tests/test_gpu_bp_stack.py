@@ -195,7 +195,8 @@ def test_scales(ctx, torch_dev):
             assert np.abs(got[s] - ref[s]).max() < 400 * 1.5e-45, v
 
 
-@pytest.mark.parametrize("storage,hot", [("f32", 1e8), ("f32", 1e20), ("f32", 3e38), ("bf16", 1e14), ("f16", 65504.0)])
+@pytest.mark.parametrize("storage,hot", [("f32", 3e4), ("f32", 1e6), ("f32", 1e8), ("f32", 1e20), ("f32", 3e38),
+                                         ("bf16", 1e9), ("bf16", 1e14), ("f16", 65504.0)])
 def test_large_sample_stays_local(ctx, torch_dev, storage, hot):
     """One large finite sample (angle 0, first detector entry) reaches the first column of voxels and leaves the
     precision of the others, in its slice and in its neighbours, as the interpolating kernel has it.  f16 storage
@@ -208,6 +209,20 @@ def test_large_sample_stays_local(ctx, torch_dev, storage, hot):
     got, ref = (t[:, :, 2:].double().cpu().numpy() for t in _both(ctx, torch_dev, x, storage))
     for s in range(33):
         assert rel_l2(got[s], ref[s]) < 1e-5, s
+
+
+@pytest.mark.parametrize("hot,matrix", [(2.0 ** 20 * 1.5, True), (2.0 ** 22 * 1.5, False)])
+def test_range_of_the_matrix_cores(ctx, torch_dev, hot, matrix):
+    """Samples of size 1 to 2 beside one of 2^20 stay on the matrix cores: their floor is 2^-40 of 2^21 at most,
+    2^-19 of a sample, and the errors of the 4 P samples of a voxel have random signs; beside 2^22 they leave."""
+    import torch
+    x = _stack(torch_dev, 64, 300, 400, seed=16)  # enough tiles that neither kernel splits the angles
+    x = torch.sign(x) * (1.0 + x.abs() % 1.0)
+    x[9, 0, 0] = hot
+    got, ref = _both(ctx, torch_dev, x, axis_pos=200.0)
+    assert torch.equal(got, ref) != matrix
+    exact = oracle.bp_texture_f64(x[9].cpu().numpy(), axis_pos=200.0)[:, 2:]
+    assert rel_l2(got[9, :, 2:].cpu().numpy(), exact) < 2.0 ** -19 + rel_l2(ref[9, :, 2:].cpu().numpy(), exact)
 
 
 def test_small_part_beside_large(ctx, torch_dev):

@@ -19,9 +19,11 @@
 //
 // The floor is absolute, so one large sample would take the precision of its
 // whole slice.  A slice of which more than 1 / 64 of the non-zero samples lie
-// below kSmall (where the floor leaves fewer bits than stated above) is left to
-// the interpolating kernel with its unit, as is one that holds an Inf or a NaN.
-// Noise puts 2e-5 of the samples there.
+// below kSmall is left to the interpolating kernel with its unit, as is one that
+// holds an Inf or a NaN.  At kSmall the floor is 2^-18 (4e-6) of a sample in f32
+// storage; half a slice of noise free samples can lie between that and the full 22
+// bits (2^-17 of the maximum) where a small object's filtered rows fall off, and
+// 6e-3 of it below.  Noise puts 1e-6 of the samples there.
 #include "ufomi_internal.h"
 
 #include <algorithm>
@@ -36,8 +38,9 @@ constexpr int kSub = 32;     // slices per stored row
 constexpr int kRow = kSub * 2;             // bytes of one plane's row of one detector entry
 constexpr int kPlane = kSpan * kRow;       // bytes of one staged plane of one angle
 constexpr int kParChunk = 64;              // angles per parameter chunk
-// Scaled samples below this keep fewer than 22 bits (f32 storage), 8 bits (bf16); f16 ones are exact.
-template <typename T> constexpr float kSmall = 0.125f;
+// Scaled samples below this, 2^-21 of the slice's maximum in f32 storage, keep fewer than 18 bits; in
+// bf16 fewer than their 8; f16 ones are exact.
+template <typename T> constexpr float kSmall = 0x1p-7f;
 template <> constexpr float kSmall<__hip_bfloat16> = 0x1p-17f;
 template <> constexpr float kSmall<__half> = 0.0f;
 constexpr unsigned kSmallShare = 64;

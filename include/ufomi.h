@@ -178,8 +178,8 @@ void ufomi_bp_params_init(ufomi_bp_params *p);
  * configuration: the same result up to rounding.  Samples keep 22 bits there
  * down to 2^-17 of their slice's largest |sample| and an absolute 2^-40 of it
  * below; slices of a larger range (more than 1 / 64 of the non-zero samples
- * below 2^-21 of the largest), or with an Inf or a NaN, stay off the matrix
- * cores together with up to 63 neighbours.  No counterpart in the
+ * below 2^-21 of the largest, or 1 / 1024 below 2^-26), or with an Inf or a
+ * NaN, stay off the matrix cores together with up to 63 neighbours.  No counterpart in the
  * reference.
  */
 int ufomi_bp_configure(ufomi_ctx *ctx, int slices_per_tile, int angle_chunk, int half_staging);

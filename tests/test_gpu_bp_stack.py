@@ -195,6 +195,17 @@ def test_scales(ctx, torch_dev):
             assert np.abs(got[s] - ref[s]).max() < 400 * 1.5e-45, v
 
 
+@pytest.mark.parametrize("scale", [1e9, 1e12, 1e25])
+def test_small_columns_at_the_axis(ctx, torch_dev, scale):
+    """Voxels at the axis see only the 8 of 700 detector columns there, a share of 1/88, whatever the others hold."""
+    x = _stack(torch_dev, 16, 300, 700, seed=17)
+    x[3, :, :346] *= scale
+    x[3, :, 354:] *= scale
+    got, ref = (t[:, 348:352, 348:352].double().cpu().numpy() for t in _both(ctx, torch_dev, x, axis_pos=350.0))
+    for s in range(16):
+        assert rel_l2(got[s], ref[s]) < 1e-5, s
+
+
 @pytest.mark.parametrize("storage,hot", [("f32", 3e4), ("f32", 1e6), ("f32", 1e8), ("f32", 1e20), ("f32", 3e38),
                                          ("bf16", 1e9), ("bf16", 1e14), ("f16", 65504.0)])
 def test_large_sample_stays_local(ctx, torch_dev, storage, hot):

@@ -19,11 +19,12 @@
 //
 // The floor is absolute, so one large sample would take the precision of its
 // whole slice.  A slice of which more than 1 / 64 of the non-zero samples lie
-// below kSmall is left to the interpolating kernel with its unit, as is one that
-// holds an Inf or a NaN.  At kSmall the floor is 2^-18 (4e-6) of a sample in f32
-// storage; half a slice of noise free samples can lie between that and the full 22
-// bits (2^-17 of the maximum) where a small object's filtered rows fall off, and
-// 6e-3 of it below.  Noise puts 1e-6 of the samples there.
+// below kSmall, or 1 / 1024 a further 2^-5 below (a voxel near the axis meets a
+// few columns only), is left to the interpolating kernel with its unit, as is one
+// that holds an Inf or a NaN.  At kSmall the floor is 2^-18 (4e-6) of a sample in
+// f32 storage; half a slice of noise free samples can lie between that and the full
+// 22 bits (2^-17 of the maximum) where a small object's filtered rows fall off,
+// 6e-3 of it below and 2e-4 of it 2^-5 further.  Noise puts 1e-6 of the samples there.
 #include "ufomi_internal.h"
 
 #include <algorithm>
@@ -43,7 +44,7 @@ constexpr int kParChunk = 64;              // angles per parameter chunk
 template <typename T> constexpr float kSmall = 0x1p-7f;
 template <> constexpr float kSmall<__hip_bfloat16> = 0x1p-17f;
 template <> constexpr float kSmall<__half> = 0.0f;
-constexpr unsigned kSmallShare = 64;
+constexpr unsigned kSmallShare = 64, kTinyWeight = 16;  // samples below kSmall / 32 count 16 times
 constexpr unsigned kLeftOut = 0x7f800000u;  // from here on, a slice's word of maxbits leaves its unit out
 constexpr int kGridY = 65535;  // a grid's second axis: the angles of split_kernel, the slices of absmax_kernel
 // Row workspace of a call: as many groups as fit, one at least; a larger group takes the other path.
@@ -137,7 +138,7 @@ __global__ __launch_bounds__(256) void split_kernel(const T *__restrict__ sino, 
         const int s = g * kSub + wv * 8 + k;
         v[k] = in && s < n_slices ? to_float(sino[(long) s * pitch + (long) p * W + j]) : 0.0f;
     }
-    unsigned few = 0;  // small samples of slice wv * 8 + lane, lane < 8
+    unsigned few = 0;  // small samples of slice wv * 8 + lane, lane < 8, the smallest ones weighted
 #pragma unroll
     for (int k = 0; k < 8; k += 2) {
         unsigned hp = 0, lp = 0;
@@ -146,8 +147,10 @@ __global__ __launch_bounds__(256) void split_kernel(const T *__restrict__ sino, 
             const int s = g * kSub + wv * 8 + k + q;
             const float x = ldexpf(v[k + q], scale_exponent<PL>(maxbits[min(s, n_slices - 1)]));
             if constexpr (kSmall<T> > 0.0f) {
-                const unsigned c = __popcll(__ballot(v[k + q] != 0.0f && fabsf(x) < kSmall<T>));
-                if (lane == k + q) few = c;
+                const bool some = v[k + q] != 0.0f;
+                const unsigned c = __popcll(__ballot(some && fabsf(x) < kSmall<T>));
+                const unsigned c2 = __popcll(__ballot(some && fabsf(x) < kSmall<T> / 32));
+                if (lane == k + q) few = c + (kTinyWeight - 1) * c2;
             }
             const _Float16 h = (_Float16) x;
             hp |= (unsigned) __builtin_bit_cast(unsigned short, h) << (16 * q);

@@ -105,6 +105,39 @@ def test_one_pipeline_on_two_contexts():
     del other
 
 
+def test_threads_with_their_own_contexts():
+    """Contexts of several threads create, run and end at the same time: their lists of idle memory are apart."""
+    import threading
+    W, P, S = 320, 700, 24   # a stack for the matrix cores: blocks and a row workspace in every context
+    xs = [torch.randn(S, P, W, device="cuda") for _ in range(3)]
+    text = _text(W, "backproject")
+    main = ufomi.Context(0, torch.cuda.current_stream())
+    want = [ufo_tasks.Pipeline(text).run(main, x, out_bytes=4 * S * W * W)[0].clone() for x in xs]
+    torch.cuda.synchronize()
+    bad = []
+
+    def work(i):
+        try:
+            st = torch.cuda.Stream()
+            for _ in range(4):
+                ctx = ufomi.Context(0, st)
+                with torch.cuda.stream(st):
+                    for _ in range(3):
+                        got = ufo_tasks.Pipeline(text).run(ctx, xs[i], out_bytes=4 * S * W * W)[0]
+                        if not torch.equal(got, want[i]):
+                            bad.append(i)
+                ctx.close()
+        except Exception as e:  # reported by the main thread
+            bad.append(repr(e))
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(3)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join(60)
+    assert not bad and not any(t.is_alive() for t in threads)
+
+
 def _fill(leave):
     """A buffer that leaves about `leave` bytes of the device free."""
     torch.cuda.synchronize()
